@@ -486,6 +486,171 @@ __global__ __launch_bounds__(256) void gemm_nn_kernel(int m, int n, int k, T alp
         }
 }
 
+// C = alpha op(A) op(B) + beta C for outputs too small to give every CU a
+// 64 x 64 tile: the k loop is split over the NW = 8 waves of a workgroup and
+// the waves' partial tiles are summed, in wave order, through LDS.
+//   What bounds such a product is one workgroup's serial k loop (1024 x 64 x
+// 1024 FP32 on 16 workgroups: 35 us, 64 steps of load, barrier, 16 MFMAs),
+// not the chip.  Splitting k inside the workgroup keeps one launch and a
+// fixed order of summation, with no workspace; the tile is 16 MT x 16 NT,
+// chosen so that the grid covers the CUs.
+//   Every wave loads its MFMA operands straight from global memory (the
+// operands of so small a product sit in L2, and no two waves of a workgroup
+// share one), three 16-k chunks ahead.  Step s of a chunk takes
+// k = 4 (lane / 16) + s as in gemm_nn_kernel, so an operand whose k runs
+// along memory is one 16-byte load a lane (two for FP64) when VEC (its rows
+// 16-byte aligned) and four element loads otherwise; one whose rows run along
+// memory is four loads of 16 consecutive elements.
+//   Addresses are clamped into the operands; only the last, partial chunk
+// masks its k, in both operands.  `lower` as in gemm_nn_kernel.
+//   Measured against the 64 x 64 tiles: FP64 Cholesky n = 8192, whose block
+// columns go through it, 12.17 -> 9.49 ms; mixed Cholesky n = 4096 with 64
+// right-hand sides 6.33 -> 3.56 ms (with the column norms'); FP64 LU n = 500
+// 1.96 -> 1.82 ms.
+constexpr int KS_WAVES = 8;
+template <class T, int MT, int NT, bool TA, bool TB, bool VEC>
+__global__ __launch_bounds__(64 * KS_WAVES) void gemm_ksplit_kernel(int m, int n, int k, T alpha,
+                                                                    const T *__restrict__ A, int64_t lda,
+                                                                    const T *__restrict__ B, int64_t ldb, T beta,
+                                                                    T *__restrict__ C, int64_t ldc, int tiles_m,
+                                                                    int tiles_n, BatchStrides bs, int lower) {
+    constexpr int NW = KS_WAVES, NREG = MT * NT * 4, PER = (NREG + NW - 1) / NW;
+    typedef typename Acc<T>::type V;
+    __shared__ T red[NW][NREG][64];
+    if (gridDim.y > 1) {
+        const int zk = (int)blockIdx.y / bs.nb1, zp = (int)blockIdx.y - zk * bs.nb1;
+        A += zk * bs.a2 + zp * bs.a1;
+        B += zk * bs.b2 + zp * bs.b1;
+        C += zk * bs.c2 + zp * bs.c1;
+    }
+    int tm, tn;
+    tile_of(tiles_m, tiles_n, lower != 0, tm, tn);
+    const int m0 = tm * 16 * MT, n0 = tn * 16 * NT;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lr = lane & 15, lk = lane >> 4;
+
+    // the C values of the registers this wave will sum: wave, wave + NW, ...
+    T cold[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int e = wave + q * NW;
+        const int a = e / (4 * NT), b = (e >> 2) % NT, r = e & 3;
+        const int gi = min(m0 + a * 16 + acc_row<T>(lk, r), m - 1), gj = min(n0 + b * 16 + lr, n - 1);
+        cold[q] = (beta != T(0) && e < NREG) ? C[(int64_t)gi * ldc + gj] : T(0);
+    }
+
+    struct Frag {
+        T a[MT][4], b[NT][4];
+    };
+    const T *pa[MT], *pb[NT];
+#pragma unroll
+    for (int a = 0; a < MT; ++a) {
+        const int64_t i = min(m0 + a * 16 + lr, m - 1);
+        pa[a] = TA ? A + i : A + i * lda;
+    }
+#pragma unroll
+    for (int b = 0; b < NT; ++b) {
+        const int64_t j = min(n0 + b * 16 + lr, n - 1);
+        pb[b] = TB ? B + j * ldb : B + j;
+    }
+    auto operand = [&](const T *p, int64_t ld, bool along, int64_t k0, T(&f)[4]) {
+        if (!along) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) f[s] = p[(k0 + s) * ld];
+        } else if constexpr (VEC) {
+            constexpr int E = V16<T>::N;
+#pragma unroll
+            for (int v = 0; v < 4 / E; ++v) {
+                const typename V16<T>::type x = *reinterpret_cast<const typename V16<T>::type *>(p + k0 + v * E);
+#pragma unroll
+                for (int q = 0; q < E; ++q) f[v * E + q] = x[q];
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) f[s] = p[k0 + s];
+        }
+    };
+    auto load = [&](Frag &f, int chunk) {
+        const int64_t k0 = (int64_t)chunk * 16 + 4 * lk;
+#pragma unroll
+        for (int a = 0; a < MT; ++a) operand(pa[a], lda, !TA, k0, f.a[a]);
+#pragma unroll
+        for (int b = 0; b < NT; ++b) operand(pb[b], ldb, TB, k0, f.b[b]);
+    };
+    V acc[MT][NT];
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < NT; ++b) acc[a][b] = V{0, 0, 0, 0};
+    auto products = [&](const Frag &f) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int a = 0; a < MT; ++a)
+#pragma unroll
+                for (int b = 0; b < NT; ++b) acc[a][b] = mfma16x16x4(f.a[a][s], f.b[b][s], acc[a][b]);
+    };
+
+    // whole chunks: a contiguous range per wave
+    const int full = k / 16, q0 = full / NW, r0 = full % NW;
+    const int c0 = wave * q0 + min(wave, r0), cnt = q0 + (wave < r0 ? 1 : 0);
+    if (cnt > 0) {
+        Frag f[3];
+#pragma unroll
+        for (int u = 0; u < 3; ++u) load(f[u], c0 + min(u, cnt - 1));
+        int i = 0;
+        for (; i + 3 <= cnt; i += 3)
+#pragma unroll
+            for (int u = 0; u < 3; ++u) {
+                products(f[u]);
+                load(f[u], c0 + min(i + u + 3, cnt - 1));
+                __builtin_amdgcn_sched_barrier(0);  // the loads stay here, three chunks ahead of their use
+            }
+        if (cnt - i > 0) products(f[0]);
+        if (cnt - i > 1) products(f[1]);
+    }
+    if ((k & 15) != 0 && wave == NW - 1) {
+        Frag f;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int64_t kk = (int64_t)full * 16 + 4 * lk + s, kc = kk < k ? kk : k - 1;
+#pragma unroll
+            for (int a = 0; a < MT; ++a) {
+                const T x = TA ? pa[a][kc * lda] : pa[a][kc];
+                f.a[a][s] = kk < k ? x : T(0);
+            }
+#pragma unroll
+            for (int b = 0; b < NT; ++b) {
+                const T x = TB ? pb[b][kc] : pb[b][kc * ldb];
+                f.b[b][s] = kk < k ? x : T(0);
+            }
+        }
+        products(f);
+    }
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < NT; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) red[wave][(a * NT + b) * 4 + r][lane] = acc[a][b][r];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        const int e = wave + q * NW;
+        if (e >= NREG) continue;
+        T sum = red[0][e][lane];
+#pragma unroll
+        for (int x = 1; x < NW; ++x) sum += red[x][e][lane];
+        const int a = e / (4 * NT), b = (e >> 2) % NT, r = e & 3;
+        const int gi = m0 + a * 16 + acc_row<T>(lk, r), gj = n0 + b * 16 + lr;
+        if (gi < m && gj < n && (!lower || gj <= gi)) {
+            T v = alpha * sum;
+            if (beta != T(0)) v += beta * cold[q];
+            C[(int64_t)gi * ldc + gj] = v;
+        }
+    }
+}
+
 // ---------------------------------------------------------------- BF16 tiles
 //
 // C (FP32) = alpha op(A) op(B) + beta C on v_mfma_f32_16x16x32_bf16 (FP32
@@ -772,6 +937,57 @@ bool nn_ok(bool ta, bool tb, int64_t n, int64_t k, const T *A, int64_t lda, cons
            bs.a1 % E == 0 && bs.a2 % E == 0 && bs.b1 % E == 0 && bs.b2 % E == 0;
 }
 
+// Tile shapes of the plain (non-batched, non-SYRK) GEMM dispatch.
+enum GemmTile { TILE_DEFAULT = 0, TILE_64x64 = 1, TILE_128x64 = 2, TILE_128x128 = 3 };
+thread_local int t_tile_override = TILE_DEFAULT;
+
+template <class T, int MT, int NT, bool VEC>
+void launch_ksplit(hipStream_t s, bool ta, bool tb, int m, int n, int k, T alpha, const T *A, int64_t lda, const T *B,
+                   int64_t ldb, T beta, T *C, int64_t ldc, int lower, int batch, const BatchStrides &bs) {
+    const int tiles_m = (int)cdiv(m, 16 * MT), tiles_n = (int)cdiv(n, 16 * NT);
+    const dim3 grid(lower ? lower_tiles(tiles_m, tiles_n) : tiles_m * tiles_n, (unsigned)batch);
+#define LMX_KSPLIT_CASE(TA_, TB_)                                                                               \
+    hipLaunchKernelGGL((gemm_ksplit_kernel<T, MT, NT, TA_, TB_, VEC>), grid, dim3(64 * KS_WAVES), 0, s, m, n, k, \
+                       alpha, A, lda, B, ldb, beta, C, ldc, tiles_m, tiles_n, bs, lower)
+    if (!ta && !tb)
+        LMX_KSPLIT_CASE(false, false);
+    else if (!ta && tb)
+        LMX_KSPLIT_CASE(false, true);
+    else if (ta && !tb)
+        LMX_KSPLIT_CASE(true, false);
+    else
+        LMX_KSPLIT_CASE(true, true);
+#undef LMX_KSPLIT_CASE
+    LMX_LAUNCH_CHECK();
+}
+
+// gemm_ksplit_kernel with the largest tile that still gives KS_FILL
+// workgroups (one a CU), else the smallest.
+constexpr int64_t KS_FILL = 256;
+constexpr int KS_MIN_K = 48;
+template <class T>
+void gemm_ksplit(hipStream_t s, bool ta, bool tb, int m, int n, int k, T alpha, const T *A, int64_t lda, const T *B,
+                 int64_t ldb, T beta, T *C, int64_t ldc, int lower, int batch, const BatchStrides &bs) {
+    // 16-byte loads along k: every row of an operand whose k runs along
+    // memory starts on a 16-byte boundary (its chunks then do too)
+    constexpr int E = V16<T>::N;
+    auto al = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
+    const bool vec = (ta || (al(A) && lda % E == 0 && bs.a1 % E == 0 && bs.a2 % E == 0)) &&
+                     (!tb || (al(B) && ldb % E == 0 && bs.b1 % E == 0 && bs.b2 % E == 0));
+    const int64_t t16 = cdiv(m, 16), t32 = cdiv(m, 32), u32 = cdiv(n, 32);
+#define LMX_KSPLIT(MT_, NT_)                                                                                    \
+    (vec ? launch_ksplit<T, MT_, NT_, true>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower, batch, bs) \
+         : launch_ksplit<T, MT_, NT_, false>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower, batch,    \
+                                             bs))
+    if ((lower ? t32 * u32 / 2 : t32 * u32) * batch >= KS_FILL)
+        LMX_KSPLIT(2, 2);
+    else if (!lower && t16 * u32 * batch >= KS_FILL)
+        LMX_KSPLIT(1, 2);
+    else
+        LMX_KSPLIT(1, 1);
+#undef LMX_KSPLIT
+}
+
 template <class T, int BM, int BN, int BK>
 void launch_tile(hipStream_t s, bool ta, bool tb, int m, int n, int k, T alpha, const T *A,
                  int64_t lda, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, int lower = 0,
@@ -779,6 +995,15 @@ void launch_tile(hipStream_t s, bool ta, bool tb, int m, int n, int k, T alpha, 
                  bool nn_sharing = false) {
     int tiles_m = (int)cdiv(m, BM), tiles_n = (int)cdiv(n, BN);
     dim3 grid(lower ? lower_tiles(tiles_m, tiles_n) : tiles_m * tiles_n, (unsigned)batch), block(256);
+    // Fewer 64 x 64 tiles than CUs: the split-k kernel (KS_MIN_K: with two
+    // 16-k chunks most of its waves would have nothing to do).
+    if constexpr (BM == 64 && BN == 64) {
+        if (lds_footprint == 0 && t_tile_override == TILE_DEFAULT && k >= KS_MIN_K &&
+            (int64_t)grid.x * batch < KS_FILL) {
+            gemm_ksplit<T>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower, batch, bs);
+            return;
+        }
+    }
     // lds_footprint: the LDS one workgroup should hold in all (its tiles plus
     // an unused reserve), so that fewer workgroups share a CU; 0 = no reserve.
     // A GEMM that shares its CUs with FP32 panel workgroups keeps the first
@@ -812,9 +1037,6 @@ void launch_tile(hipStream_t s, bool ta, bool tb, int m, int n, int k, T alpha, 
     LMX_LAUNCH_CHECK();
 }
 
-// Tile shapes of the plain (non-batched, non-SYRK) GEMM dispatch.
-enum GemmTile { TILE_DEFAULT = 0, TILE_64x64 = 1, TILE_128x64 = 2, TILE_128x128 = 3 };
-
 // The autotuned table (gemm_tiles.inc, written by tune_gemm.py): for an
 // element size and ranges of ceil(log2) of m, n and k, the tile that timed
 // fastest on MI355X.  Shapes no rule covers take the fixed rule below.
@@ -830,8 +1052,6 @@ int ceil_log2(int64_t v) {
     while (((int64_t)1 << b) < v) ++b;
     return b;
 }
-
-thread_local int t_tile_override = TILE_DEFAULT;
 
 int table_tile(int bytes, int64_t m, int64_t n, int64_t k) {
     if (t_tile_override != TILE_DEFAULT) return t_tile_override;
