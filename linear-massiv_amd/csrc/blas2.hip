@@ -88,8 +88,10 @@ __global__ __launch_bounds__(256) void norm_inf_rows_kernel(const double *__rest
 
 // out[c] = max_i |X[i][c]| for an n x ncols block: a workgroup covers
 // COLMAX_ROWS rows and 64 columns (blockIdx.y), reduces in LDS, and issues
-// one atomic per column.
-constexpr int COLMAX_ROWS = 1024;
+// one atomic per column.  32 rows a workgroup: 8 loads a thread, all in
+// flight (1024 rows a workgroup left 4 of them for n = 4096, each thread
+// waiting for 256 loads: 67 us for 4096 x 64).
+constexpr int COLMAX_ROWS = 32;
 __global__ __launch_bounds__(256) void colmax_kernel(const double *__restrict__ X, int64_t ldx, int64_t n,
                                                      int ncols, double *__restrict__ out) {
     __shared__ double part[4][64];
@@ -97,11 +99,14 @@ __global__ __launch_bounds__(256) void colmax_kernel(const double *__restrict__ 
     const int c = blockIdx.y * 64 + cl;
     const int64_t r0 = (int64_t)blockIdx.x * COLMAX_ROWS;
     double m = 0.0;
-    if (c < ncols)
-        for (int64_t i = r0 + q; i < n && i < r0 + COLMAX_ROWS; i += 4) {
-            double v = fabs(X[i * ldx + c]);
-            if (!(v <= m)) m = v;  // keeps NaN
-        }
+    if (c < ncols) {
+        double v[COLMAX_ROWS / 4];
+#pragma unroll
+        for (int u = 0; u < COLMAX_ROWS / 4; ++u) v[u] = fabs(X[min(r0 + q + 4 * u, n - 1) * ldx + c]);
+#pragma unroll
+        for (int u = 0; u < COLMAX_ROWS / 4; ++u)
+            if (!(v[u] <= m)) m = v[u];  // keeps NaN; a row past the end repeats the last one
+    }
     part[q][cl] = m;
     __syncthreads();
     if (q == 0 && c < ncols) {

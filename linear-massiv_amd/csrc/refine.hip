@@ -30,18 +30,29 @@ constexpr double EPS64 = 2.220446049250313e-16;
 
 // norms layout: [0] ||A||, [1..1+k) ||b_c||, [1+k..1+2k) ||x_c||, [1+2k..1+3k) ||r_c||,
 // [1+3k] eta, [2+3k] all-columns-pass flag (1.0 / 0.0)
+// One wave: a lane per column forms its ratio (one thread going through the
+// columns waited for three loads a column: 13 us for 64), and the columns'
+// ratios are then compared in order.
 __global__ void eta_kernel(double *norms, int k, double crit) {
-    if (threadIdx.x != 0) return;
-    double nA = norms[0], eta = 0.0, pass = 1.0;
-    for (int c = 0; c < k; ++c) {
-        double nb = norms[1 + c], nx = norms[1 + k + c], nr = norms[1 + 2 * k + c];
-        double den = nA * nx + nb;
-        double e = den > 0.0 ? nr / den : (nr > 0.0 ? __builtin_huge_val() : 0.0);
-        if (!(e <= eta)) eta = e;  // keeps NaN
-        if (!(nr <= crit * nA * nx)) pass = 0.0;
+    const int lane = threadIdx.x;
+    const double nA = norms[0];
+    double eta = 0.0;
+    bool pass = true;
+    for (int c0 = 0; c0 < k; c0 += 64) {
+        const int c = min(c0 + lane, k - 1);
+        const double nb = norms[1 + c], nx = norms[1 + k + c], nr = norms[1 + 2 * k + c];
+        const double den = nA * nx + nb;
+        const double e = den > 0.0 ? nr / den : (nr > 0.0 ? __builtin_huge_val() : 0.0);
+        pass = pass && __ballot(!(nr <= crit * nA * nx)) == 0;
+        for (int q = 0; q < min(64, k - c0); ++q) {
+            const double eq = bcast_lane(e, q);
+            if (!(eq <= eta)) eta = eq;  // keeps NaN
+        }
     }
-    norms[1 + 3 * k] = eta;
-    norms[2 + 3 * k] = pass;
+    if (lane == 0) {
+        norms[1 + 3 * k] = eta;
+        norms[2 + 3 * k] = pass ? 1.0 : 0.0;
+    }
 }
 
 
