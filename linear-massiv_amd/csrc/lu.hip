@@ -2,27 +2,31 @@
 // LU solve, for row-major matrices.
 //
 // Panel kernel (getf2_panel_kernel): the m x kb panel (kb <= 32) is spread
-// over P concurrent workgroups of 512 rows each (FP32: 4 waves, two rows a
-// thread; FP64: 8 waves, one row a thread), rows held in registers.  Per
+// over P concurrent workgroups of 512 rows each, rows held in registers.  Per
 // column j:
-//   1. each workgroup finds its candidate max |a_ij| over rows i >= j (ties:
-//      lowest row, NaN never chosen -- the rule of rawPivotSearch,
-//      src/.../Internal/Kernel.hs:1541-1556; or, for the generic lu, the
-//      highest row among equal magnitudes -- maximumBy keeps the later of
-//      two equal elements, src/.../Solve/LU.hs:128-135): DPP wave
+//   1. each wave, then each workgroup, finds its candidate max |a_ij| over
+//      rows i >= j (ties: lowest row, NaN never chosen -- the rule of
+//      rawPivotSearch, src/.../Internal/Kernel.hs:1541-1556; or, for the
+//      generic lu, the highest row among equal magnitudes -- maximumBy keeps
+//      the later of two equal elements, src/.../Solve/LU.hs:128-135): DPP
 //      reductions and ballots, then one LDS exchange between the waves;
-//   2. it publishes the candidate (value, row, full row data) in slot j%2,
-//      and workgroup 0 publishes row j, each word tagged with the column;
-//   3. every workgroup polls all P records, reduces them to the pivot p,
-//      swaps rows j and p, and all rows i > j get l = a_ij / a_pj (a
-//      division, as the reference) and the rank-1 update of the remaining
-//      panel columns.
+//   2. several workgroups publish their candidates, each word tagged with the
+//      column, poll each other's and pick the pivot p;
+//   3. rows j and p exchange positions, all rows i > j get
+//      l = a_ij / a_pj (a division, as the reference) and column j + 1; the
+//      rank-1 update of the other columns follows while column j + 1 is
+//      searched.
 // The current column always sits in register 0..3: after every 4 columns
 // the row's registers rotate left by 4, so the column loop needs no dynamic
 // register indexing.  At the end every workgroup derives the panel's
 // row-move list from the pivots and applies it to the other columns of the
 // outer panel (and the permutation vector) with one parallel gather, and
 // solves U12 = L11^{-1} B12 for the columns to the right of the panel.
+//   One column took 4.4 us in FP64 at 16 workgroups (n = 8192) when the
+// candidates' whole rows went through the exchange and the whole update lay
+// between two of them; FP64 LU n = 2048 / 4096 / 8192 / 16384: 9.5 / 20.2 /
+// 46.7 / 153 -> 6.5 / 14.0 / 35.6 / 141 ms, FP32 6.7 / 14.4 / 31.3 / 78.6 ->
+// 5.8 / 12.4 / 27.4 / 72.5 ms.
 //
 // Driver (getrf_impl): outer panels of NB = 256 columns, each factored as
 // eight 32-column sub-panels (panel kernel, then A22 -= L21 U12 inside the
@@ -50,26 +54,28 @@ constexpr int NB_OUTER = 256; // outer panel width (k of the trailing GEMM)
 constexpr long SPIN_LIMIT = 1L << 22;
 
 // Cross-workgroup records of the panel kernel.  Every word is 64 bits: a
-// 32-bit payload and, in the upper half, the tag base + j + 1 of the column
-// it belongs to, written with one device-coherent store; a reader polls a
-// word until its tag matches, so the poll is the load and no flag is needed.
-// Tags grow over the whole factorisation (the records are zeroed once per
-// getrf) and records are double-buffered by column parity.
-//   workgroup record: value (WPV words), row, pad, row data
-//   row-j record:     pad, pad, row data
+// 32-bit payload and, in the upper half, (base + j + 1) << POS_BITS | pos: the
+// tag of the column it belongs to and the position of the row it offers,
+// written with one device-coherent store; a reader polls a word until its tag
+// matches, so the poll is the load and no flag is needed.  Tags grow over the
+// whole factorisation (the records are zeroed once per getrf) and records are
+// double-buffered by column parity.
+//   key record:  a workgroup's offer for column j (three numbers), in a
+//                64-byte line of its own (32 workgroups polling packed keys:
+//                0.96 us an exchange, keys a line apart: 0.73 us)
+//   row record:  the whole row it offers
+constexpr int POS_BITS = 16;
+constexpr int POS_NONE = (1 << POS_BITS) - 1;  // above every position of a panel
 template <class T>
 struct PanelRec {
     static constexpr int WPV = sizeof(T) / 4;
-    static constexpr int DATA = WPV + 2;  // data offset (even for doubles)
-    static constexpr int W = DATA + KB * WPV;                  // words per workgroup record
-    static constexpr int DDATA = 2;
-    static constexpr int DW = DDATA + KB * WPV;                // words of the row-j record
-    static constexpr int TOTAL = MAXP * W + DW;
+    static constexpr int KEYW = 8;         // words from key to key
+    static constexpr int ROWW = KB * WPV;  // words of a row record
 };
 template <class T>
 struct PanelSync {
-    // the P workgroup records, then the row-j record (at P * W)
-    unsigned long long rec[2][PanelRec<T>::TOTAL];
+    unsigned long long key[2][MAXP][PanelRec<T>::KEYW];
+    unsigned long long row[2][MAXP][PanelRec<T>::ROWW];
     unsigned error;
     unsigned pad[63];
 };
@@ -90,58 +96,79 @@ __device__ inline unsigned word_of(T v, int h) {
                       : (unsigned)(__builtin_bit_cast(unsigned long long, v) >> 32);
 }
 
+template <class T>
+__device__ inline T value_of(const unsigned long long *words) {
+    if constexpr (sizeof(T) == 4)
+        return __builtin_bit_cast(T, (unsigned)words[0]);
+    else
+        return __builtin_bit_cast(T, (words[0] & 0xffffffffull) | (words[1] << 32));
+}
+
 constexpr int PG = 4;  // columns per register rotation
 
 // Shape of the partial-pivoting panel kernel's workgroup (PANEL_ROWS rows):
-// 8 waves of one row a thread.  A wave's rows are consecutive: row block q
-// of a wave is rows 64 q .. 64 q + 63 of its 64 RPT.  (Two rows a thread in
-// 4 waves, and a one-row panel held to 85 registers, both let a panel
-// workgroup share its CU with two workgroups of the FP32 lookahead GEMM;
-// both measured slower beside that GEMM.)
+// 4 waves hold the rows, two a thread (64 apart), a wave's 128 rows
+// consecutive; with several workgroups a fifth wave talks to the others.
+// What a column costs is latency and LDS: a wave that reads the pivot row
+// from LDS for all its lanes takes 64 of the 128 bytes a clock for as long
+// whatever its lanes hold, so two rows a thread halve that (one row a thread
+// in 8 waves: 1400 cycles to read the row and start the update).
 template <class T>
 struct PanelShape {
-    static constexpr int RPT = 1;               // rows per thread
-    static constexpr int PT = PANEL_ROWS / RPT;  // threads
-    static constexpr int PW = PT / 64;           // waves
-    static constexpr int MIN_WAVES_PER_SIMD = 2;
+    static constexpr int WROWS = 128;  // rows of a wave
+    static constexpr int WAVES = PANEL_ROWS / WROWS;
+    // FP32: at most 128 registers, so that a wave of the FP32 lookahead GEMM
+    // finds room beside two panel waves on a SIMD (with 256, the panels waited
+    // for CUs without any: FP32 LU n = 16384 80 against 72 ms)
+    static constexpr int MIN_WAVES_PER_SIMD = sizeof(T) == 4 ? 4 : 2;
 };
 
-// Per-thread state of the panel kernel: R rows of the panel in registers,
-// in the rotated frame (register c holds column j0 + c of the current
-// group).
-template <class T, int R>
-struct PanelRows {
-    T v[R][KB];
-    int row[R];
-};
-
-// Columns a pass of the panel kernel's closing row gather: the U12 block
-// of a pass (KB x GCOLS) shares LDS with the poll payloads.
+// Per-thread state of the panel kernel: its rows in registers, in the rotated
+// frame (register c holds column j0 + c of the current group).  Rows stay
+// where they are: an interchange exchanges the rows' positions, and a row is
+// stored at the position it ended at.  While column j is searched, column j is
+// up to date and the columns after it are up to column j - 2; l holds the
+// rows' multipliers of column j - 1.
 template <class T>
-constexpr int gather_cols() {
-    return 64;
-}
+struct PanelRows {
+    T v[2][KB];
+    T l[2];
+    int pos[2];
+};
 
-// LDS of the panel kernel.  What is written before a column's first
-// barrier (wave slots, row j) is double-buffered by column parity; the poll
-// payloads are written after it and read before the next column's, so one
-// buffer serves.
+// The communicating wave: words of the previous column's pivot row in flight,
+// and from which record.
+struct PanelComm {
+    unsigned long long rw = 0;
+    int src = 0;
+    bool failed = false;  // a wait ran out: no further waiting
+};
+
+// LDS of the panel kernel.  What one workgroup alone reads after the one
+// barrier of a column is double-buffered by column parity; with several
+// workgroups prow[0] and the results are written and read on opposite sides
+// of a barrier.
 template <class T>
 struct PanelLds {
-    static constexpr int NW = PanelShape<T>::PW;
-    alignas(16) T slot_data[2][NW][KB];  // each wave's best row
-    T slot_val[2][NW];
-    int slot_row[2][NW];
-    T drow[2][KB];                 // row j (single workgroup)
+    static constexpr int NW = PanelShape<T>::WAVES;
+    // columns of the rows a pass of panel_rows_move takes (64 bytes), and the
+    // row stride that keeps 16-byte accesses of 16 rows on distinct banks
+    static constexpr int TCOLS = 64 / (int)sizeof(T), TLD = 80 / (int)sizeof(T);
+    // per wave: its candidate's magnitude (two words) and position, its value
+    // in column j, in column j + 1 (up to column j - 2) and its multiplier of
+    // column j - 1
+    int slot_hi[2][NW], slot_lo[2][NW], slot_pos[2][NW];
+    T slot_v[2][NW], slot_n[2][NW], slot_l[2][NW];
+    T res[2];  // pivot and its row's column j + 1
+    int res_p;
     int pivs[KB];
-    T l11[KB][KB];                 // the panel's unit-lower L11: row j recorded at column j
-    union {
-        alignas(8) unsigned pay[PanelRec<T>::TOTAL];  // polled record payloads (several workgroups)
-        alignas(16) T b12[KB][gather_cols<T>()];      // closing gather: B12, then U12
-    };
     int mv_dst[2 * KB];  // the rows that move (panel-relative) ...
     int mv_src[2 * KB];  // ... and the original row each one receives
     int mv_cnt;
+    alignas(16) T prow[2][KB + PG];  // the pivot row, then PG zeros
+    alignas(16) T stage[KB];         // a row on its way to its record
+    alignas(16) T l11[KB][KB];       // column k of the panel's unit-lower L11 at l11[k]
+    alignas(16) T tile[NW][64][TLD];  // panel rows on their way in and out
 };
 
 // Tie rules of the pivot search: the lowest row among equal magnitudes
@@ -188,203 +215,340 @@ __device__ __forceinline__ int tie_index(unsigned long long mask) {
     return TL ? 63 - __builtin_clzll(mask) : __builtin_ctzll(mask);
 }
 
-// One column (j = j0 + U) of the panel: pivot search, interchange, scaling
-// and rank-1 update of the rest of the panel.
+// |x| as a pair of integers ordered like it (hi, then lo); hi is 0 for a row
+// that is not searched and for NaN (never chosen), and above all others for a
+// NaN in row j (which keeps row j, as rawPivotSearch does).  DPP maxima of
+// integers take one instruction a step, those of doubles five.
+__device__ __forceinline__ void magnitude(float x, bool live, bool rowj, int &hi, int &lo) {
+    const unsigned b = __float_as_uint(x) & 0x7fffffffu;
+    hi = !live ? 0 : (b <= 0x7f800000u ? (int)(b + 1u) : (rowj ? INT_MAX : 0));
+    lo = 0;
+}
+__device__ __forceinline__ void magnitude(double x, bool live, bool rowj, int &hi, int &lo) {
+    const unsigned b = (unsigned)__double2hiint(x) & 0x7fffffffu;
+    hi = !live ? 0 : (!isnan(x) ? (int)(b + 1u) : (rowj ? INT_MAX : 0));
+    lo = (int)((unsigned)__double2loint(x) ^ 0x80000000u);
+}
+// The lane that offers the largest magnitude, by the tie rule on the
+// positions; -1 if none offers any.
+template <class T, bool TL>
+__device__ __forceinline__ int largest_lane(int hi, int lo, int pos) {
+    const int mh = wave_max_int(hi);
+    if (mh == 0) return -1;
+    unsigned long long mk = __ballot(hi == mh);
+    if (mk & (mk - 1)) {
+        bool in = hi == mh;
+        if constexpr (sizeof(T) == 8) {
+            const int ml = wave_max_int(in ? lo : INT_MIN);
+            in = in && lo == ml;
+        }
+        const int mp = TieRule<TL>::wave_pick(in ? pos : TieRule<TL>::NONE);
+        mk = __ballot(in && pos == mp);
+    }
+    return __builtin_ctzll(mk);
+}
+
+// ---- a column of the panel
+//
+// Between the search of column j and that of column j + 1 lies only what
+// column j + 1 needs: the pivot, the multipliers and column j + 1 of the
+// rows.  A candidate is therefore offered as three numbers: its value in
+// column j, its value in column j + 1 before column j - 1's update, and its
+// multiplier of column j - 1; with element j + 1 of column j - 1's pivot row
+// they give the pivot row's element j + 1.  The rank-1 update of the columns
+// from j + 1 on by column j - 1 (registers C1 ..) runs beside that, a column
+// late.
+
+// a or b, both in registers: selected as lvalues, the compiler keeps the
+// rows' arrays in memory to select between addresses.
+template <class T>
+__device__ __forceinline__ T pick(bool c, T a, T b) {
+    asm volatile("" : "+v"(a), "+v"(b));
+    return c ? a : b;
+}
+
+// Each wave offers its candidate; returns it as 2 lane + row, -1 for none.
 template <class T, int U, bool TL>
-__device__ __forceinline__ void panel_column(PanelRows<T, PanelShape<T>::RPT> &st, PanelLds<T> &L, int j0, int kb,
-                                             int m, int P, PanelSync<T> *__restrict__ sy, unsigned base, int k0,
-                                             int32_t *__restrict__ ipiv, int &local_info, bool &failed) {
-    typedef PanelShape<T> S;
-    constexpr int NR = S::RPT;
-    typedef PanelRec<T> R;
-    typedef TieRule<TL> Tie;
-    const int j = j0 + U;
-    if (j >= kb) return;
-    const int w = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int par = j & 1;
-    // 1. this wave's candidate: max |a_ij| over its rows i >= j (fmax skips
-    //    NaN), then the tie rule's row among those attaining it (row block
-    //    q of a wave precedes block q + 1, lanes ascend within a block);
-    //    the owning lane writes that row to the wave slot
-    bool live[NR];
-    T a[NR];
-    T tmax = T(-1);
-#pragma unroll
-    for (int q = 0; q < NR; ++q) {
-        live[q] = st.row[q] >= j && st.row[q] < m;
-        a[q] = live[q] ? fabs(st.v[q][U]) : T(-1);
-        tmax = fmax(tmax, a[q]);
+__device__ __forceinline__ int panel_offer(const PanelRows<T> &st, PanelLds<T> &L, int j, int m) {
+    constexpr int C1 = U + 1;
+    const int par = j & 1, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int hi, lo, h1, l1;
+    magnitude(st.v[0][U], st.pos[0] >= j && st.pos[0] < m, st.pos[0] == j, hi, lo);
+    magnitude(st.v[1][U], st.pos[1] >= j && st.pos[1] < m, st.pos[1] == j, h1, l1);
+    const bool q = h1 > hi || (h1 == hi && (l1 > lo || (l1 == lo && TieRule<TL>::better(st.pos[1], st.pos[0]))));
+    hi = q ? h1 : hi;
+    lo = q ? l1 : lo;
+    const int pos = q ? st.pos[1] : st.pos[0];
+    const T v = pick(q, st.v[1][U], st.v[0][U]), n = pick(q, st.v[1][C1], st.v[0][C1]), l = pick(q, st.l[1], st.l[0]);
+    const int wl = largest_lane<T, TL>(hi, lo, pos);
+    if (lane == max(wl, 0)) {
+        L.slot_hi[par][wave] = wl < 0 ? 0 : hi;
+        L.slot_lo[par][wave] = lo;
+        L.slot_pos[par][wave] = wl < 0 ? POS_NONE : pos;
+        L.slot_v[par][wave] = v;
+        L.slot_n[par][wave] = n;
+        L.slot_l[par][wave] = l;
     }
-    const T wmax = wave_max(tmax);
-    int wl = -1, wq = 0;
-#pragma unroll
-    for (int qq = 0; qq < NR; ++qq) {
-        const int q = TL ? NR - 1 - qq : qq;
-        const unsigned long long mk = __ballot(a[q] == wmax && a[q] >= T(0));
-        if (wl < 0 && mk != 0) {
-            wl = tie_index<TL>(mk);
-            wq = q;
-        }
-    }
-    if (lane == wl) {
-#pragma unroll
-        for (int c = 0; c < KB; ++c) {
-            T x = st.v[0][c];
-#pragma unroll
-            for (int q = 1; q < NR; ++q) x = wq == q ? st.v[q][c] : x;
-            L.slot_data[par][wave][c] = x;
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < NR; ++q)
-        if (st.row[q] == j) {
-#pragma unroll
-            for (int c = 0; c < KB; ++c) L.drow[par][c] = st.v[q][c];
-        }
-    if (lane == 0) {
-        // a wave with no candidate offers -1, so no slot holds a NaN
-        L.slot_val[par][wave] = wl < 0 ? T(-1) : wmax;
-        L.slot_row[par][wave] = wl < 0 ? Tie::NONE : w * PANEL_ROWS + wave * 64 * NR + wq * 64 + wl;
-    }
-    __syncthreads();
-    // 2. this workgroup's candidate: lane x reads slot x; waves hold
-    //    ascending rows, so the tie rule over rows is the one over waves
-    const T sv = lane < S::PW ? L.slot_val[par][lane] : T(-1);
-    const T best = wave_max(sv);
-    const int bw = tie_index<TL>(__ballot(lane < S::PW && sv == best && best >= T(0)));
-    const int brow = bw < 0 ? Tie::NONE : L.slot_row[par][bw];
-    int p;
-    const T *prow;
-    const T *drow;
-    if (P == 1) {
-        drow = L.drow[par];
-        // a NaN at row j keeps row j, as rawPivotSearch does
-        if (bw < 0 || isnan(drow[U])) {
-            p = j;
-            prow = drow;
-        } else {
-            p = brow;
-            prow = L.slot_data[par][bw];
-        }
-    } else {
-        const unsigned tg = base + (unsigned)j + 1u;
-        // The records' base, opaque to the compiler: every address below is
-        // formed here, in the column, rather than hoisted out of the column
-        // loop into registers held across all of it.
-        unsigned long long *rbase = sy->rec[par];
-        asm volatile("" : "+v"(rbase));
-        // 3. publish this workgroup's record (and row j from workgroup 0):
-        //    lane e of wave 0 writes word e
-        if (wave == 0) {
-            unsigned long long *rec = rbase + w * R::W;
-            const unsigned *data = reinterpret_cast<const unsigned *>(L.slot_data[par][bw < 0 ? 0 : bw]);
-            for (int e = lane; e < R::W; e += 64) {
-                const unsigned dv = data[max(e - R::DATA, 0)];
-                const unsigned hv = e < R::WPV ? word_of(best, e) : (e == R::WPV ? (unsigned)brow : 0u);
-                const unsigned pl = e >= R::DATA ? (bw < 0 ? 0u : dv) : hv;
-                xstore(rec + e, tagword(pl, tg));
-            }
-            if (w == 0) {
-                const unsigned *dd = reinterpret_cast<const unsigned *>(L.drow[par]);
-                for (int e = lane; e < R::DW; e += 64) {
-                    const unsigned dv = dd[max(e - R::DDATA, 0)];
-                    xstore(rbase + P * R::W + e, tagword(e >= R::DDATA ? dv : 0u, tg));
-                }
-            }
-        }
-        // 4. poll every record: all loads in flight first, then the
-        //    stragglers one by one
-        constexpr int NPOLL = (R::TOTAL + S::PT - 1) / S::PT;
-        const int total = P * R::W + R::DW;
-        unsigned long long wv[NPOLL];
-#pragma unroll
-        for (int i = 0; i < NPOLL; ++i) {
-            const int e = t + i * S::PT;
-            if (e < total) {
-                wv[i] = xload(rbase + e);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < NPOLL; ++i) {
-            const int e = t + i * S::PT;
-            if (e < total) {
-                const unsigned long long *wp = rbase + e;
-                long spins = 0;
-                while ((unsigned)(wv[i] >> 32) != tg && !failed) {
-                    __builtin_amdgcn_s_sleep(1);
-                    if ((++spins & 255) == 0 && xload(&sy->error) != 0u) failed = true;
-                    if (spins > SPIN_LIMIT) {
-                        xstore(&sy->error, 1u);
-                        failed = true;
-                    }
-                    wv[i] = xload(wp);
-                }
-                L.pay[e] = (unsigned)wv[i];
-            }
-        }
-        __syncthreads();
-        // 5. the pivot: largest value over the workgroups; workgroups hold
-        //    ascending rows, so the tie rule over rows is the one over
-        //    workgroups.  Every wave reduces the P records itself (lane x
-        //    reads record x).  Record values are -1 or a magnitude, never NaN.
-        const unsigned *pay = L.pay;
-        const T xv = lane < P ? *reinterpret_cast<const T *>(pay + lane * R::W) : T(-1);
-        const T gb = wave_max(xv);
-        const int gw = tie_index<TL>(__ballot(lane < P && xv == gb && gb >= T(0)));
-        drow = reinterpret_cast<const T *>(pay + P * R::W + R::DDATA);
-        if (gw < 0 || isnan(drow[U])) {
-            p = j;
-            prow = drow;
-        } else {
-            p = (int)pay[gw * R::W + R::WPV];
-            prow = reinterpret_cast<const T *>(pay + gw * R::W + R::DATA);
-        }
-    }
-    // row j of L11: the pivot row's multipliers of columns k < j (final
-    // since column k; register (k - j0) mod KB in the rotated frame)
-    if (t < j) L.l11[j][t] = prow[(t - j0) & (KB - 1)];
-    // 6. interchange rows j and p
-    if (p != j) {
-#pragma unroll
-        for (int q = 0; q < NR; ++q) {
-            if (st.row[q] == p) {
-#pragma unroll
-                for (int c = 0; c < KB; ++c) st.v[q][c] = drow[c];
-            } else if (st.row[q] == j) {
-#pragma unroll
-                for (int c = 0; c < KB; ++c) st.v[q][c] = prow[c];
-            }
-        }
-    }
-    if (t == 0) L.pivs[j] = p;
-    if (w == 0 && t == 0) ipiv[k0 + j] = k0 + p;
-    // 7. multipliers (a division, as the reference) and the rank-1 update
-    //    of the panel columns after j.  The pivot row is read from LDS in
-    //    one batch first.  Registers past KB - j0 hold the finished columns
-    //    (rotated to the end) and are skipped in blocks of PG; registers of
-    //    columns past kb (a narrow last panel) are padding that is updated
-    //    but never stored.
+    return wl < 0 ? -1 : 2 * wl + __builtin_amdgcn_readlane((int)q, wl);
+}
+
+// The wave with the workgroup's best offer (-1: none): every group of four
+// lanes compares the four.
+template <class T, bool TL>
+__device__ __forceinline__ int panel_best(const PanelLds<T> &L, int par) {
+    static_assert(PanelShape<T>::WAVES == 4, "a quad of lanes compares the waves' offers");
+    const int x = threadIdx.x & 3;
+    const int hi = L.slot_hi[par][x], lo = L.slot_lo[par][x], pos = L.slot_pos[par][x];
+    int mh = max(hi, dpp_i<0xB1, 0xF>(hi));
+    mh = max(mh, dpp_i<0x4E, 0xF>(mh));
+    unsigned mk = (unsigned)__ballot(hi == mh && hi > 0) & 15u;
+    if (mk & (mk - 1)) return largest_lane<T, TL>((threadIdx.x & 63) < 4 ? hi : 0, lo, pos);
+    return mk ? __builtin_ctz(mk) : -1;
+}
+
+// acc -= l p, in place: with the FMA left to the compiler, a row updated
+// under a branch is computed into other registers and copied back.
+__device__ __forceinline__ void fnma(double &acc, double l, double p) {
+    asm("v_fma_f64 %0, -%1, %2, %0" : "+v"(acc) : "v"(l), "v"(p));
+}
+__device__ __forceinline__ void fnma(float &acc, float l, float p) {
+    asm("v_fma_f32 %0, -%1, %2, %0" : "+v"(acc) : "v"(l), "v"(p));
+}
+
+// Column j - 1 on whole rows: row j - 1 of L11 and the update of the columns
+// after j.  Registers from KB - j0 on hold finished columns (rotated to the
+// end): their blocks of PG take multipliers and a pivot row of zeros, which
+// leaves them as they are without a branch a block (branches made the
+// compiler spill).  Registers of columns past kb (a narrow last panel) and
+// rows past m are padding, updated but never stored.
+template <class T, int U>
+__device__ __forceinline__ void panel_update(PanelRows<T> &st, PanelLds<T> &L, bool update, const T *prow, int j,
+                                             int j0) {
+    constexpr int SH = U == 0 ? PG : 0, C1 = U + 1, B1 = (C1 + PG - 1) / PG * PG;
+    const int t = threadIdx.x;
+    if (t < j - 1) L.l11[t][j - 1] = prow[(t - (j0 - SH)) & (KB - 1)];
+    if (!update) return;
     T pr[KB];
 #pragma unroll
-    for (int c = U; c < KB; ++c) pr[c] = prow[c];
-    const T piv = pr[U];
+    for (int c = C1; c < B1; ++c) pr[c] = prow[(c + SH) & (KB - 1)];
+#pragma unroll
+    for (int b = B1; b < KB; b += PG) {
+        const int src = b < KB - j0 ? (b + SH) & (KB - 1) : KB;
+#pragma unroll
+        for (int e = 0; e < PG; ++e) pr[b + e] = prow[src + e];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        if (st.pos[i] >= j) {
+#pragma unroll
+            for (int c = C1; c < B1; ++c) fnma(st.v[i][c], st.l[i], pr[c]);
+#pragma unroll
+            for (int b = B1; b < KB; b += PG) {
+                const T l = b < KB - j0 ? st.l[i] : T(0);
+#pragma unroll
+                for (int e = 0; e < PG; ++e) fnma(st.v[i][b + e], l, pr[b + e]);
+            }
+        }
+}
+
+// From column j's pivot: the interchange of positions, the multipliers (a
+// division, as the reference) and column j + 1.  val: the pivot and its row's
+// column j + 1.
+template <class T, int U>
+__device__ __forceinline__ void panel_pivot(PanelRows<T> &st, PanelLds<T> &L, const T (&val)[2], int p, int j, int kb,
+                                            int k0, int w, int32_t *__restrict__ ipiv, int &local_info) {
+    constexpr int C1 = U + 1;
+    const T piv = val[0];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int pos = st.pos[i];
+        st.pos[i] = pos == p ? j : (pos == j ? p : pos);
+    }
     if (piv != T(0)) {
 #pragma unroll
-        for (int q = 0; q < NR; ++q)
-            if (live[q] && st.row[q] > j) {
-                const T l = st.v[q][U] / piv;
-                st.v[q][U] = l;
-#pragma unroll
-                for (int b = (U + 1) / PG * PG; b < KB; b += PG)
-                    if (b < KB - j0) {
-#pragma unroll
-                        for (int e = 0; e < PG; ++e)
-                            if (b + e > U) st.v[q][b + e] = fma(-l, pr[b + e], st.v[q][b + e]);
-                    }
+        for (int i = 0; i < 2; ++i)
+            if (st.pos[i] > j) {
+                const T l = st.v[i][U] / piv;
+                st.v[i][U] = l;
+                st.l[i] = l;
+                if (j + 1 < kb) fnma(st.v[i][C1], l, val[1]);
             }
     } else if (local_info == 0) {
         local_info = k0 + j + 1;
     }
+    if (threadIdx.x == 0) {
+        L.pivs[j] = p;
+        if (w == 0) ipiv[k0 + j] = k0 + p;
+    }
+}
+
+// A column of a panel that fits one workgroup: one barrier, after which every
+// wave picks the pivot itself.  `update`: column j - 1 has multipliers; on
+// return, column j has.
+template <class T, int U, bool TL>
+__device__ __forceinline__ void panel_column(PanelRows<T> &st, PanelLds<T> &L, bool &update, int j0, int kb, int m,
+                                             int k0, int32_t *__restrict__ ipiv, int &local_info) {
+    constexpr int SH = U == 0 ? PG : 0, C1 = U + 1;
+    const int j = j0 + U;
+    if (j >= kb) return;
+    const int par = j & 1;
+    panel_offer<T, U, TL>(st, L, j, m);
+    __syncthreads();
+    const T *prow = L.prow[par ^ 1];
+    const int bw = panel_best<T, TL>(L, par);  // row j is always offered
+    const int p = L.slot_pos[par][bw];
+    T val[2] = {L.slot_v[par][bw], L.slot_n[par][bw]};
+    if (update) val[1] = fma(-L.slot_l[par][bw], prow[(C1 + SH) & (KB - 1)], val[1]);
+    if (j > 0) panel_update<T, U>(st, L, update, prow, j, j0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        if (st.pos[i] == p) {
+#pragma unroll
+            for (int c = 0; c < KB; ++c) L.prow[par][c] = st.v[i][c];
+        }
+    panel_pivot<T, U>(st, L, val, p, j, kb, k0, 0, ipiv, local_info);
+    update = val[0] != T(0);
+}
+
+// ---- panels of several workgroups: one exchange a column
+//
+// The rows' waves as above; the fifth wave publishes the workgroup's offer,
+// polls everyone's, picks the pivot and fetches its whole row, which is
+// needed only behind the next column's offers.  Barriers: the offers are in
+// LDS; column j - 1's pivot row is; column j's pivot is.
+// (Whole rows in the polled records instead, one poll for everything, no
+// second fetch: 17 KB polled by every workgroup and column at 32 workgroups,
+// and the whole update on the way from one exchange to the next.)
+
+// Polls N words until they all carry tag tg, all of them each time round (a
+// word at a time waits a round trip for each); v holds a first reading.
+// Bounded: on a time-out the error flag is set and nothing waits any more.
+template <int N, class T>
+__device__ __forceinline__ void panel_await(const unsigned long long *words, unsigned long long (&v)[N], unsigned tg,
+                                            PanelSync<T> *sy, bool &failed) {
+    long spins = 0;
+    for (;;) {
+        bool there = true;
+#pragma unroll
+        for (int i = 0; i < N; ++i) there = there && (unsigned)(v[i] >> (32 + POS_BITS)) == tg;
+        if (there || failed) return;
+        if ((++spins & 255) == 0 && xload(&sy->error) != 0u) failed = true;
+        if (spins > SPIN_LIMIT) {
+            xstore(&sy->error, 1u);
+            failed = true;
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = xload(words + i);
+    }
+}
+
+// The whole pivot row of column j - 1 into LDS (communicating wave).
+template <class T>
+__device__ __forceinline__ void panel_receive_row(PanelLds<T> &L, PanelComm &cm, int j, PanelSync<T> *sy,
+                                                  unsigned base) {
+    constexpr int ROWW = PanelRec<T>::ROWW;
+    const int lane = threadIdx.x & 63;
+    if (lane < ROWW) {
+        unsigned long long v[1] = {cm.rw};
+        panel_await(sy->row[(j - 1) & 1][cm.src] + lane, v, base + (unsigned)j, sy, cm.failed);
+        reinterpret_cast<unsigned *>(L.prow[0])[lane] = (unsigned)v[0];
+    }
+    cm.failed = __any(cm.failed);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+}
+
+// The communicating wave's side of all columns.
+template <class T, bool TL>
+__device__ __forceinline__ void panel_communicate(PanelLds<T> &L, int kb, int P, PanelSync<T> *__restrict__ sy,
+                                                  unsigned base) {
+    typedef PanelRec<T> R;
+    constexpr int WPV = R::WPV;
+    const int lane = threadIdx.x & 63;
+    PanelComm cm;
+    bool update = false;
+    for (int j = 0; j < kb; ++j) {
+        const unsigned tg = base + (unsigned)j + 1u;
+        const unsigned long long *key = sy->key[j & 1][min(lane, P - 1)];
+        unsigned long long kw[3 * WPV];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 3 * WPV; ++i) kw[i] = xload(key + i);
+        if (j > 0) panel_receive_row(L, cm, j, sy, base);
+        // element j + 1 of that row, in the frame of column j - 1
+        const T c1 = update ? L.prow[0][(j + 1 - (j - 1) / PG * PG) & (KB - 1)] : T(0);
+        __syncthreads();
+        // the pivot: the largest of the workgroups' offers
+        panel_await(key, kw, tg, sy, cm.failed);
+        cm.failed = __any(cm.failed);
+        const T v0 = value_of<T>(kw);
+        T v1 = value_of<T>(kw + WPV);
+        if (update) v1 = fma(-value_of<T>(kw + 2 * WPV), c1, v1);
+        const int pos = (int)(unsigned)(kw[0] >> 32) & POS_NONE;
+        int mh, ml;
+        magnitude(v0, lane < P && pos != POS_NONE, true, mh, ml);  // a NaN is offered for row j only
+        int gw = largest_lane<T, TL>(mh, ml, pos);                  // row j is always offered
+        if (cm.failed) gw = -1;
+        const int gl = max(gw, 0);
+        if (lane == gl) {
+            L.res_p = gw < 0 ? j : pos;
+            L.res[0] = gw < 0 ? T(0) : v0;
+            L.res[1] = v1;
+        }
+        cm.src = gl;
+        cm.rw = xload(sy->row[j & 1][gl] + min(lane, R::ROWW - 1));
+        update = gw >= 0 && bcast_lane(v0, gl) != T(0);
+        __syncthreads();
+    }
+    panel_receive_row(L, cm, kb, sy, base);
+}
+
+// A column on the side of the rows.
+template <class T, int U, bool TL>
+__device__ __forceinline__ void panel_column_multi(PanelRows<T> &st, PanelLds<T> &L, bool &update, int j0, int kb,
+                                                   int m, int w, PanelSync<T> *__restrict__ sy, unsigned base, int k0,
+                                                   int32_t *__restrict__ ipiv, int &local_info) {
+    typedef PanelRec<T> R;
+    constexpr int C1 = U + 1, WPV = R::WPV;
+    const int j = j0 + U;
+    if (j >= kb) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int par = j & 1;
+    const unsigned tg = (base + (unsigned)j + 1u) << POS_BITS;
+    const int mine = panel_offer<T, U, TL>(st, L, j, m);
+    const bool q = mine > 0 && (mine & 1) != 0;
+    __syncthreads();
+    const int bw = panel_best<T, TL>(L, par);
+    const bool owner = max(bw, 0) == wave, holder = owner && lane == max(mine, 0) / 2;
+    if (owner) {
+        const T v = pick(q, st.v[1][U], st.v[0][U]), n = pick(q, st.v[1][C1], st.v[0][C1]),
+                l = pick(q, st.l[1], st.l[0]);
+        const unsigned hi = tg | (unsigned)(bw < 0 ? POS_NONE : (q ? st.pos[1] : st.pos[0]));
+        if (holder) {
+            unsigned long long *key = sy->key[par][w];
+#pragma unroll
+            for (int h = 0; h < WPV; ++h) {
+                xstore(key + h, tagword(word_of(v, h), hi));
+                xstore(key + WPV + h, tagword(word_of(n, h), hi));
+                xstore(key + 2 * WPV + h, tagword(word_of(l, h), hi));
+            }
+        }
+    }
+    __syncthreads();
+    if (j > 0) panel_update<T, U>(st, L, update, L.prow[0], j, j0);
+    if (owner) {
+        if (holder) {
+#pragma unroll
+            for (int c = 0; c < KB; ++c) L.stage[c] = pick(q, st.v[1][c], st.v[0][c]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (lane < R::ROWW)
+            xstore(sy->row[par][w] + lane, tagword(reinterpret_cast<const unsigned *>(L.stage)[lane], tg));
+    }
+    __syncthreads();
+    const T val[2] = {L.res[0], L.res[1]};
+    panel_pivot<T, U>(st, L, val, L.res_p, j, kb, k0, w, ipiv, local_info);
+    update = val[0] != T(0);
 }
 
 // 16-byte vectors of panel row elements.
@@ -415,198 +579,231 @@ struct PanelGather {
     int u12;
 };
 
-// At most 128 VGPRs (four waves a SIMD), so that GEMM waves of the other
-// stream still find registers on the panel's CUs.
-template <class T, bool TL>
-__global__ __launch_bounds__(PanelShape<T>::PT)
-__attribute__((amdgpu_waves_per_eu(PanelShape<T>::MIN_WAVES_PER_SIMD))) void getf2_panel_kernel(int m, int kb, T *__restrict__ A, int64_t lda,
-                                                          int k0, int32_t *__restrict__ ipiv,
-                                                          int32_t *__restrict__ info,
-                                                          PanelSync<T> *__restrict__ sy, int P,
-                                                          unsigned base, PanelGather<T> gx) {
+// The wave's 128 panel rows between memory and registers, 64 bytes of every
+// row at a time through LDS, so that an access covers 16 rows (a row a lane,
+// 64 lines an instruction, took 4 us a panel to store).  Rows past m load row
+// m - 1 and are not stored; a row goes to its position.
+template <class T, bool STORE>
+__device__ __forceinline__ void panel_rows_move(PanelRows<T> &st, PanelLds<T> &L, T *A, int64_t lda, int r0, int m) {
+    typedef typename RowVec<T>::type V;
+    constexpr int VE = 16 / sizeof(T), TC = PanelLds<T>::TCOLS;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    T(*tile)[PanelLds<T>::TLD] = L.tile[wave];
+    T *base = A + lane % 4 * VE;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        // access i covers rows 16 i .. 16 i + 15 of these 64, four lanes a row
+        int row[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = 16 * i + lane / 4;
+            row[i] = STORE ? __shfl(st.pos[q], e) : min(r0 + 64 * q + e, m - 1);
+        }
+#pragma unroll
+        for (int c0 = 0; c0 < KB; c0 += TC) {
+            V x[4];
+            if (!STORE) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[i] = *reinterpret_cast<const V *>(base + (int64_t)row[i] * lda + c0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) *reinterpret_cast<V *>(&tile[16 * i + lane / 4][lane % 4 * VE]) = x[i];
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+#pragma unroll
+            for (int c = 0; c < TC; c += VE) {
+                V *p = reinterpret_cast<V *>(&tile[lane][c]);
+                V y;
+                if (STORE) {
+#pragma unroll
+                    for (int e = 0; e < VE; ++e) y[e] = st.v[q][c0 + c + e];
+                    *p = y;
+                } else {
+                    y = *p;
+#pragma unroll
+                    for (int e = 0; e < VE; ++e) st.v[q][c0 + c + e] = y[e];
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            if (STORE) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    x[i] = *reinterpret_cast<const V *>(&tile[16 * i + lane / 4][lane % 4 * VE]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (row[i] < m) *reinterpret_cast<V *>(base + (int64_t)row[i] * lda + c0) = x[i];
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+    }
+}
+
+template <class T, bool TL, bool MULTI>
+__global__ __launch_bounds__(64 * (PanelShape<T>::WAVES + (MULTI ? 1 : 0)))
+__attribute__((amdgpu_waves_per_eu(PanelShape<T>::MIN_WAVES_PER_SIMD))) void getf2_panel_kernel(
+    int m, int kb, T *__restrict__ A, int64_t lda, int k0, int32_t *__restrict__ ipiv, int32_t *__restrict__ info,
+    PanelSync<T> *__restrict__ sy, int P, unsigned base, PanelGather<T> gx) {
     critical_path_priority();
     typedef PanelShape<T> S;
-    const int w = blockIdx.x, t = threadIdx.x;
+    const int w = MULTI ? (int)blockIdx.x : 0, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const bool rows = !MULTI || wave < S::WAVES;  // a wave that holds rows
     __shared__ PanelLds<T> L;
-    PanelRows<T, S::RPT> st;
-    // A full-width panel whose rows start on 16-byte boundaries moves each
-    // row in 16-byte vectors (a quarter of the address work of 4-byte ones)
-    typedef typename RowVec<T>::type V;
-    constexpr int VE = 16 / sizeof(T);
+    PanelRows<T> st;
+    // A full-width panel whose rows start on 16-byte boundaries moves whole
+    // rows in 16-byte vectors
     const bool vec = kb == KB && (reinterpret_cast<uintptr_t>(A) & 15) == 0 && ((lda * (int64_t)sizeof(T)) & 15) == 0;
+    const int r0 = w * PANEL_ROWS + wave * S::WROWS;
 #pragma unroll
-    for (int q = 0; q < S::RPT; ++q) {
-        st.row[q] = w * PANEL_ROWS + (t >> 6) * 64 * S::RPT + q * 64 + (t & 63);
+    for (int q = 0; q < 2; ++q) {
+        st.pos[q] = rows ? r0 + 64 * q + lane : m;
+        st.l[q] = T(0);
+    }
+    if (rows) {
         if (vec) {
-            const T *src = A + (int64_t)st.row[q] * lda;
-#pragma unroll
-            for (int c = 0; c < KB; c += VE) {
-                V x = {};
-                if (st.row[q] < m) x = *reinterpret_cast<const V *>(src + c);
-#pragma unroll
-                for (int e = 0; e < VE; ++e) st.v[q][c + e] = x[e];
-            }
+            panel_rows_move<T, false>(st, L, A, lda, r0, m);
         } else {
 #pragma unroll
-            for (int c = 0; c < KB; ++c)
-                st.v[q][c] = (st.row[q] < m && c < kb) ? A[(int64_t)st.row[q] * lda + c] : T(0);
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int c = 0; c < KB; ++c)
+                    st.v[q][c] = (st.pos[q] < m && c < kb) ? A[(int64_t)st.pos[q] * lda + c] : T(0);
         }
     }
+    if (t < 2 * PG) L.prow[t / PG][KB + t % PG] = T(0);
     int local_info = 0;
-    bool failed = false;
+    bool update = false;
     int groups = 0;
-    for (int j0 = 0; j0 < kb; j0 += PG) {
-        panel_column<T, 0, TL>(st, L, j0, kb, m, P, sy, base, k0, ipiv, local_info, failed);
-        panel_column<T, 1, TL>(st, L, j0, kb, m, P, sy, base, k0, ipiv, local_info, failed);
-        panel_column<T, 2, TL>(st, L, j0, kb, m, P, sy, base, k0, ipiv, local_info, failed);
-        panel_column<T, 3, TL>(st, L, j0, kb, m, P, sy, base, k0, ipiv, local_info, failed);
-        // rotate: the next group's first column moves to register 0
+    if (!rows) {
+        panel_communicate<T, TL>(L, kb, P, sy, base);
+    } else {
+        for (int j0 = 0; j0 < kb; j0 += PG) {
+            if constexpr (MULTI) {
+                panel_column_multi<T, 0, TL>(st, L, update, j0, kb, m, w, sy, base, k0, ipiv, local_info);
+                panel_column_multi<T, 1, TL>(st, L, update, j0, kb, m, w, sy, base, k0, ipiv, local_info);
+                panel_column_multi<T, 2, TL>(st, L, update, j0, kb, m, w, sy, base, k0, ipiv, local_info);
+                panel_column_multi<T, 3, TL>(st, L, update, j0, kb, m, w, sy, base, k0, ipiv, local_info);
+            } else {
+                panel_column<T, 0, TL>(st, L, update, j0, kb, m, k0, ipiv, local_info);
+                panel_column<T, 1, TL>(st, L, update, j0, kb, m, k0, ipiv, local_info);
+                panel_column<T, 2, TL>(st, L, update, j0, kb, m, k0, ipiv, local_info);
+                panel_column<T, 3, TL>(st, L, update, j0, kb, m, k0, ipiv, local_info);
+            }
+            // rotate: the next group's first column moves to register 0
 #pragma unroll
-        for (int q = 0; q < S::RPT; ++q) {
-            T keep[PG];
+            for (int q = 0; q < 2; ++q) {
+                T keep[PG];
 #pragma unroll
-            for (int c = 0; c < PG; ++c) keep[c] = st.v[q][c];
+                for (int c = 0; c < PG; ++c) keep[c] = st.v[q][c];
 #pragma unroll
-            for (int c = 0; c < KB - PG; ++c) st.v[q][c] = st.v[q][c + PG];
+                for (int c = 0; c < KB - PG; ++c) st.v[q][c] = st.v[q][c + PG];
 #pragma unroll
-            for (int c = 0; c < PG; ++c) st.v[q][KB - PG + c] = keep[c];
+                for (int c = 0; c < PG; ++c) st.v[q][KB - PG + c] = keep[c];
+            }
+            ++groups;
         }
-        ++groups;
     }
+    // the last column's row of L11
     __syncthreads();
-
+    if (t < kb - 1) L.l11[t][kb - 1] = L.prow[MULTI ? 0 : (kb - 1) & 1][(t - (kb - 1) / PG * PG) & (KB - 1)];
     // After the rotations register s holds column (s + PG*groups) % KB
     // (column s itself for a full-width panel: KB / PG rotations).
-    const int shift = (PG * groups) % KB;
+    if (rows) {
+        if (vec) {
+            panel_rows_move<T, true>(st, L, A, lda, r0, m);
+        } else {
+            const int shift = (PG * groups) % KB;
 #pragma unroll
-    for (int q = 0; q < S::RPT; ++q)
-        if (st.row[q] < m) {
-            T *dst = A + (int64_t)st.row[q] * lda;
-            if (vec) {
+            for (int q = 0; q < 2; ++q)
+                if (st.pos[q] < m) {
+                    T *dst = A + (int64_t)st.pos[q] * lda;
 #pragma unroll
-                for (int c = 0; c < KB; c += VE) {
-                    V x;
-#pragma unroll
-                    for (int e = 0; e < VE; ++e) x[e] = st.v[q][c + e];
-                    *reinterpret_cast<V *>(dst + c) = x;
+                    for (int s2 = 0; s2 < KB; ++s2) {
+                        const int c = (s2 + shift) % KB;
+                        if (c < kb) dst[c] = st.v[q][s2];
+                    }
                 }
-            } else {
-#pragma unroll
-                for (int s2 = 0; s2 < KB; ++s2) {
-                    int c = (s2 + shift) % KB;
-                    if (c < kb) dst[c] = st.v[q][s2];
-                }
-            }
         }
-    // The row interchanges on the other columns.  Every workgroup knows
-    // every pivot (L.pivs), so each one derives the move list itself:
+    }
+    // The row interchanges on the other columns.  Every workgroup knows every
+    // pivot (L.pivs), so each one derives the move list itself:
     //  a. the rows that move: panel rows 0 .. min(kb, m) - 1, then each pivot
     //     row below the panel's diagonal block once, in the order of the
-    //     columns that first chose it (lane j of wave 0 takes column j's
-    //     pivot; a ballot gives its place in the list);
-    //  b. the original row each of them receives: lane e holds the tag of
-    //     the row at position mv_dst[e] and the kb interchanges are
-    //     replayed on those tags;
-    //  c. the gather itself, gather_cols() columns a pass, each column read
-    //     by one workgroup before it is written; for B12's columns one
-    //     thread a column then solves U12 = L11^{-1} B12 (unit lower,
-    //     x_i -= l_ik x_k with k ascending for every i) between the reads
-    //     and the writes.
+    //     columns that first chose it (lane j takes column j's pivot; a
+    //     ballot gives its place in the list);
+    //  b. the original row each of them receives: every lane follows its row
+    //     back through the interchanges, the last one first;
+    //  c. the gather itself, 64 columns a wave, a column a lane with its rows
+    //     in registers: every row is read before one is written, and B12's
+    //     columns are solved between, U12 = L11^{-1} B12 (unit lower,
+    //     x_i -= l_ik x_k with k ascending for every i).
     const int nd = min(kb, m);
     if (t < 64) {
         const int pj = t < kb ? L.pivs[t] : -1;
         bool keep = t < kb && pj >= kb;
 #pragma unroll
-        for (int x = 0; x < KB; ++x)
-            if (x < kb) keep = keep && !(x < t && L.pivs[x] == pj);
+        for (int x = 0; x < KB; ++x) {
+            const int px = __builtin_amdgcn_readlane(pj, x);
+            keep = keep && !(x < t && px == pj);
+        }
         const unsigned long long mask = __ballot(keep);
+        const int cnt = nd + __popcll(mask);
         if (t < nd) L.mv_dst[t] = t;
         if (keep) L.mv_dst[nd + __popcll(mask & ((1ull << t) - 1ull))] = pj;
-        if (t == 0) L.mv_cnt = nd + __popcll(mask);
-    }
-    __syncthreads();
-    const int cnt = L.mv_cnt;
-    if (t < 64) {
-        const int pos = t < cnt ? L.mv_dst[t] : -1;
-        const int pv = t < kb ? L.pivs[t] : 0;
-        int tag = pos;
-        for (int jj = 0; jj < kb; ++jj) {
-            const int p = __builtin_amdgcn_readlane(pv, jj);
-            if (p == jj) continue;
-            // the lane holding position p (positions below kb are lanes)
-            const int lp = p < nd ? p : __builtin_ctzll(__ballot(pos == p));
-            const int tj = __builtin_amdgcn_readlane(tag, jj);
-            const int tp = __builtin_amdgcn_readlane(tag, lp);
-            tag = t == jj ? tp : (t == lp ? tj : tag);
-        }
-        L.mv_src[t] = t < cnt ? tag : 0;
         if (t >= cnt) L.mv_dst[t] = 0;
-        if (w == 0 && t == 0 && local_info != 0 && *info == 0) *info = local_info;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        int pos = L.mv_dst[t];
+        for (int jj = kb - 1; jj >= 0; --jj) {
+            const int p = __builtin_amdgcn_readlane(pj, jj);
+            pos = pos == jj ? p : (pos == p ? jj : pos);
+        }
+        L.mv_src[t] = t < cnt ? pos : 0;
+        if (t == 0) {
+            L.mv_cnt = cnt;
+            if (w == 0 && local_info != 0 && *info == 0) *info = local_info;
+        }
     }
     __syncthreads();
-    if (w == 0 && gx.pairs_out != nullptr && t < 64) {
-        if (t == 0) gx.pairs_out[0] = cnt;
-        gx.pairs_out[1 + t] = k0 + L.mv_dst[t];
-        gx.pairs_out[1 + 2 * KB + t] = k0 + L.mv_src[t];
+    const int cnt = L.mv_cnt, dst = L.mv_dst[lane], src = L.mv_src[lane];
+    if (w == 0 && wave == 0) {
+        if (gx.pairs_out != nullptr) {
+            if (t == 0) gx.pairs_out[0] = cnt;
+            gx.pairs_out[1 + t] = k0 + dst;
+            gx.pairs_out[1 + 2 * KB + t] = k0 + src;
+        }
+        if (gx.perm != nullptr) {
+            const int pv = gx.perm[src];
+            if (t < cnt) gx.perm[dst] = pv;
+        }
     }
+    if (!rows) return;
     const int n1 = gx.c1 - gx.c0, ncols = n1 + (gx.c3 - gx.c2);
-    constexpr int GCOLS = gather_cols<T>(), GPER = 2 * KB / (S::PT / GCOLS);  // columns a pass; moves per thread
     const bool u12 = gx.u12 != 0 && kb == KB;
-    const int lane = t & 63, wave = t >> 6;
-    // for the U12 solve: lane i holds row i of L11 (columns k < i)
-    T lrow[KB];
+    for (int c0 = (wave * P + w) * 64; c0 < ncols; c0 += S::WAVES * P * 64) {
+        const int c = c0 + lane, cc = min(c, ncols - 1);
+        T *col = gx.G + (cc < n1 ? gx.c0 + cc : gx.c2 + (cc - n1));
+        T x[2 * KB];
 #pragma unroll
-    for (int k = 0; k < KB; ++k) lrow[k] = (u12 && lane < KB && k < lane) ? L.l11[lane][k] : T(0);
-    // workgroup w takes a contiguous chunk of the columns
-    const int chunk = (ncols + P - 1) / P;
-    const int cbeg = w * chunk, cend = min(ncols, cbeg + chunk);
-    for (int cb = cbeg; cb < cend; cb += GCOLS) {
-        const int tc = t % GCOLS, cc = cb + tc, grp = t / GCOLS;
-        const int col = cc >= cend ? -1 : (cc < n1 ? gx.c0 + cc : gx.c2 + (cc - n1));
-        const bool ucol = u12 && cc >= n1 && col >= 0;  // a column of B12
-        // a wave's threads share grp, so the rows are wave-uniform
-        T val[GPER];
+        for (int e = 0; e < 2 * KB; ++e)
+            if (e < KB || e < cnt) x[e] = col[(int64_t)__builtin_amdgcn_readlane(src, e) * gx.ldg];
+        if (u12 && cc >= n1) {
 #pragma unroll
-        for (int i = 0; i < GPER; ++i) {
-            const int e = grp * GPER + i;
-            const T *src = gx.G + (int64_t)__builtin_amdgcn_readfirstlane(L.mv_src[e]) * gx.ldg;
-            val[i] = (col >= 0 && e < cnt) ? src[col] : T(0);
-            // positions 0 .. KB - 1 are the first KB entries of the list
-            if (ucol && e < KB) L.b12[e][tc] = val[i];
-        }
-        __syncthreads();
+            for (int k = 0; k < KB - 1; ++k) {
 #pragma unroll
-        for (int i = 0; i < GPER; ++i) {
-            const int e = grp * GPER + i;
-            T *dst = gx.G + (int64_t)__builtin_amdgcn_readfirstlane(L.mv_dst[e]) * gx.ldg;
-            if (col >= 0 && e < cnt && !(ucol && e < KB)) dst[col] = val[i];
-        }
-        if (u12) {
-            // U12 = L11^{-1} B12, a column per wave: lane i holds x_i, and
-            // step k broadcasts x_k (by v_readlane) to x_i -= l_ik x_k for
-            // the lanes i > k -- every x_i takes its terms in ascending k.
-            // Rows 0 .. KB - 1 are positions 0 .. KB - 1.
-            for (int q = wave; q < GCOLS; q += S::PW) {
-                const int cq = cb + q;
-                if (cq >= cend || cq < n1) continue;
-                T x = lane < KB ? L.b12[lane][q] : T(0);
-#pragma unroll
-                for (int k = 0; k < KB - 1; ++k) {
-                    const T xk = bcast_lane(x, k);
-                    x = lane > k ? fma(-lrow[k], xk, x) : x;
-                }
-                if (lane < KB) (gx.G + (int64_t)lane * gx.ldg)[gx.c2 + (cq - n1)] = x;
+                for (int i = k + 1; i < KB; ++i) x[i] = fma(-L.l11[k][i], x[k], x[i]);
+                // the next columns of L11 stay in LDS until their turn
+                if (k % 2 == 1) __builtin_amdgcn_sched_barrier(0);
             }
-            __syncthreads();  // the next pass rewrites b12
         }
-    }
-    if (w == 0 && gx.perm != nullptr) {
-        const int pv = t < cnt ? gx.perm[L.mv_src[t]] : 0;
-        __syncthreads();
-        if (t < cnt) gx.perm[L.mv_dst[t]] = pv;
+        if (c < ncols) {
+#pragma unroll
+            for (int e = 0; e < 2 * KB; ++e)
+                if (e < cnt) col[(int64_t)__builtin_amdgcn_readlane(dst, e) * gx.ldg] = x[e];
+        }
     }
 }
-
 
 // ---------------------------------------------------------------- tournament panel
 //
@@ -1233,12 +1430,18 @@ void launch_panel(hipStream_t s, int m, int kb, T *A, int64_t lda, int k0, int32
     // hardware queue of its own: each hand-over between it and the stream's
     // other kernels cost about 11 us (about 10 ms per FP32 factorisation at
     // n = 16384).
-    if (tie_last)
-        hipLaunchKernelGGL((getf2_panel_kernel<T, true>), dim3(P), dim3(PanelShape<T>::PT), 0, s, m, kb, A, lda, k0, ipiv, info,
-                           sy, P, base, gx);
+#define LMX_PANEL(TL_, MULTI_)                                                                                     \
+    hipLaunchKernelGGL((getf2_panel_kernel<T, TL_, MULTI_>), dim3(P), dim3(64 * (PanelShape<T>::WAVES + MULTI_)), 0, \
+                       s, m, kb, A, lda, k0, ipiv, info, sy, P, base, gx)
+    if (P > 1 && tie_last)
+        LMX_PANEL(true, true);
+    else if (P > 1)
+        LMX_PANEL(false, true);
+    else if (tie_last)
+        LMX_PANEL(true, false);
     else
-        hipLaunchKernelGGL((getf2_panel_kernel<T, false>), dim3(P), dim3(PanelShape<T>::PT), 0, s, m, kb, A, lda, k0, ipiv, info,
-                           sy, P, base, gx);
+        LMX_PANEL(false, false);
+#undef LMX_PANEL
     LMX_LAUNCH_CHECK();
     base += (unsigned)kb;  // sequence numbers stay monotonic across launches
 }
