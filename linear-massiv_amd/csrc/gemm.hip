@@ -884,6 +884,191 @@ bool bf16_vec_ok(bool ta, bool tb, int64_t m, int64_t n, int64_t k, const S *A, 
     return al(A) && al(B) && lda % 4 == 0 && ldb % 4 == 0 && a_ok && b_ok;
 }
 
+// ---- BF16 operands, large outputs
+//
+// BT = 256: 256 x 256 x 64 tiles, 8 waves in a 2 x 4 grid, each 128 x 64 of C on
+// v_mfma_f32_32x32x16_bf16 (a 128 x 64 wave tile reads 24 KB of LDS for 64
+// MFMAs, 0.75 of the LDS bandwidth the matrix cores leave time for; the
+// 128 x 128 tiles of 64 x 64 waves read a third more a product).  One
+// workgroup a CU: 2 x 72 KB of LDS, two buffers, one barrier a k step; the
+// next step's loads are in registers while this step's products run.
+//   Operands lie k-contiguous in LDS (row stride 144 bytes: 16-byte reads of
+// 16 rows on distinct banks).  One whose k runs along memory moves in 16-byte
+// vectors; the other is read as 4 (k) x 8 blocks of 16-byte vectors,
+// transposed in registers (v_perm on pairs) and written as 8-byte runs of k,
+// the lanes of a wave on consecutive k.
+//   For rows aligned to 16 bytes and dimensions along memory that are
+// multiples of 8.  Bound by the matrix cores and LDS: 8192^3 2.43 -> 1.21 ms
+// (453 -> 908 TF) as stored, 1.53 -> 1.05 ms with B transposed, against the
+// 128 x 128 x 32 tiles with 8-byte loads; 4096^3 370 -> 136 - 166 us.  The same
+// with 128 x 128 tiles, 4 waves of 64 x 64, two workgroups a CU, for outputs
+// that leave CUs without a tile: 2048 x 2048 x 4096 145 -> 82 us.
+typedef float f16v __attribute__((ext_vector_type(16)));
+typedef unsigned u4 __attribute__((ext_vector_type(4)));
+constexpr int BX_K = 64, BX_SK = 72;
+constexpr int64_t BX_MIN_TILES = 100;
+
+template <bool KC, int NT>
+struct BxTile {
+    u4 r[4];
+    // op(X)[row][k] is X[row ldx + k] (KC) or X[k ldx + row]; r0, k0: the
+    // tile's origin
+    __device__ __forceinline__ void load(const unsigned short *__restrict__ X, int64_t ldx, int r0, int rows, int k0,
+                                         int kdim) {
+        const int t = threadIdx.x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            int row, kk;
+            if (KC) {
+                const int e = i * NT + t;
+                row = r0 + e / 8;
+                kk = k0 + e % 8 * 8;
+            } else {
+                row = r0 + t / 16 * 8;
+                kk = k0 + t % 16 * 4 + i;
+            }
+            const bool in = row < rows && kk < kdim;
+            const unsigned short *p = KC ? X + (int64_t)row * ldx + kk : X + (int64_t)kk * ldx + row;
+            r[i] = in ? *reinterpret_cast<const u4 *>(p) : u4{0, 0, 0, 0};
+        }
+    }
+    __device__ __forceinline__ void store(unsigned short (*S)[BX_SK]) const {
+        const int t = threadIdx.x;
+        if (KC) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int e = i * NT + t;
+                *reinterpret_cast<u4 *>(&S[e / 8][e % 8 * 8]) = r[i];
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                // element q of the four k: low or high halves of word q / 2
+                const unsigned sel = q & 1 ? 0x07060302u : 0x05040100u;
+                uint2 w;
+                w.x = __builtin_amdgcn_perm(r[1][q / 2], r[0][q / 2], sel);
+                w.y = __builtin_amdgcn_perm(r[3][q / 2], r[2][q / 2], sel);
+                *reinterpret_cast<uint2 *>(&S[t / 16 * 8 + q][t % 16 * 4]) = w;
+            }
+        }
+    }
+};
+
+template <int BT, bool TA, bool TB>
+__global__ __launch_bounds__(2 * BT) void gemm_bf16_large_kernel(int m, int n, int k, float alpha,
+                                                              const unsigned short *__restrict__ A, int64_t lda,
+                                                              const unsigned short *__restrict__ B, int64_t ldb,
+                                                              float beta, float *__restrict__ C, int64_t ldc,
+                                                              int tiles_m, int tiles_n) {
+    constexpr int NT = 2 * BT, WC = BT / 64, MT = BT / 64;  // threads, waves across, 32-row blocks of a wave
+    __shared__ __attribute__((aligned(16))) unsigned short As[2][BT][BX_SK];
+    __shared__ __attribute__((aligned(16))) unsigned short Bs[2][BT][BX_SK];
+    int tm, tn;
+    tile_of(tiles_m, tiles_n, false, tm, tn);
+    const int m0 = tm * BT, n0 = tn * BT;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm0 = wave / WC * (BT / 2), wn0 = wave % WC * 64;
+    const int lr = lane & 31, lk = lane >> 5;
+    f16v acc[MT][2];
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[a][b][r] = 0.0f;
+
+    BxTile<!TA, NT> ta;
+    BxTile<TB, NT> tb;
+    const int KT = (k + BX_K - 1) / BX_K;
+    if (KT > 0) {
+        ta.load(A, lda, m0, m, 0, k);
+        tb.load(B, ldb, n0, n, 0, k);
+        ta.store(As[0]);
+        tb.store(Bs[0]);
+        __syncthreads();
+    }
+    for (int kt = 0; kt < KT; ++kt) {
+        const int cur = kt & 1;
+        const bool more = kt + 1 < KT;
+        if (more) {
+            ta.load(A, lda, m0, m, (kt + 1) * BX_K, k);
+            tb.load(B, ldb, n0, n, (kt + 1) * BX_K, k);
+        }
+#pragma unroll
+        for (int ks = 0; ks < BX_K; ks += 16) {
+            bf16x8 fa[MT], fb[2];
+#pragma unroll
+            for (int a = 0; a < MT; ++a)
+                fa[a] = *reinterpret_cast<const bf16x8 *>(&As[cur][wm0 + 32 * a + lr][ks + 8 * lk]);
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+                fb[b] = *reinterpret_cast<const bf16x8 *>(&Bs[cur][wn0 + 32 * b + lr][ks + 8 * lk]);
+#pragma unroll
+            for (int a = 0; a < MT; ++a)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[a], fb[b], acc[a][b], 0, 0, 0);
+        }
+        if (more) {
+            ta.store(As[cur ^ 1]);
+            tb.store(Bs[cur ^ 1]);
+        }
+        __syncthreads();
+    }
+    // accumulator value r of a 32 x 32 block: row 8 (r / 4) + 4 (lane / 32) + r % 4
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int gj = n0 + wn0 + 32 * b + lr;
+            if (gj >= n) continue;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int gi = m0 + wm0 + 32 * a + 8 * (r / 4) + 4 * lk + r % 4;
+                if (gi < m) {
+                    float *c = C + (int64_t)gi * ldc + gj;
+                    float v = alpha * acc[a][b][r];
+                    if (beta != 0.0f) v += beta * *c;
+                    *c = v;
+                }
+            }
+        }
+}
+
+// The tile gemm_bf16_large_kernel takes a product with, 0 where it does not:
+// every 16-byte vector has to be wholly inside or outside its operand and
+// aligned.
+int bf16_large_tile(bool ta, bool tb, int64_t m, int64_t n, int64_t k, const unsigned short *A, int64_t lda,
+                    const unsigned short *B, int64_t ldb) {
+    auto al = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
+    if (!(al(A) && al(B) && lda % 8 == 0 && ldb % 8 == 0 && (ta ? m : k) % 8 == 0 && (tb ? k : n) % 8 == 0)) return 0;
+    // rounds over the chip, one 256 x 256 tile a CU or two 128 x 128; a round
+    // of the former takes 40 / 23 of the latter's time (2048 x 4096 x 8192 NT:
+    // 206 against 160 us, one round each)
+    const int64_t t256 = cdiv(m, 256) * cdiv(n, 256), t128 = cdiv(m, 128) * cdiv(n, 128);
+    if (t128 < BX_MIN_TILES) return 0;  // the 64 x 64 tiles spread better (1024^3 NT: 15.0 against 19.3 us)
+    return 40 * cdiv(t256, 256) <= 23 * cdiv(t128, 512) ? 256 : 128;
+}
+
+template <int BT>
+void launch_bf16_large(hipStream_t s, bool ta, bool tb, int m, int n, int k, float alpha, const unsigned short *A,
+                       int64_t lda, const unsigned short *B, int64_t ldb, float beta, float *C, int64_t ldc) {
+    const int tiles_m = (int)cdiv(m, BT), tiles_n = (int)cdiv(n, BT);
+#define LMX_BX_CASE(TA_, TB_)                                                                                         \
+    hipLaunchKernelGGL((gemm_bf16_large_kernel<BT, TA_, TB_>), dim3(tiles_m *tiles_n), dim3(2 * BT), 0, s, m, n, k,   \
+                       alpha, A, lda, B, ldb, beta, C, ldc, tiles_m, tiles_n)
+    if (!ta && !tb)
+        LMX_BX_CASE(false, false);
+    else if (!ta && tb)
+        LMX_BX_CASE(false, true);
+    else if (ta && !tb)
+        LMX_BX_CASE(true, false);
+    else
+        LMX_BX_CASE(true, true);
+#undef LMX_BX_CASE
+    LMX_LAUNCH_CHECK();
+}
+
 template <class S, bool SPLIT>
 void gemm_bf16_impl(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k, float alpha, const S *A,
                     int64_t lda, const S *B, int64_t ldb, float beta, float *C, int64_t ldc, int lower,
@@ -897,6 +1082,11 @@ void gemm_bf16_impl(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64
     const bool vec = bf16_vec_ok<S>(ta, tb, m, n, k, A, lda, B, ldb);
     const int64_t big = lower ? cdiv(m, 128) * (cdiv(m, 128) + 1) / 2 : cdiv(m, 128) * cdiv(n, 128);
     const int M = (int)m, N = (int)n, K = (int)k;
+    if constexpr (sizeof(S) == 2) {
+        const int tile = lower ? 0 : bf16_large_tile(ta, tb, m, n, k, A, lda, B, ldb);
+        if (tile == 256) return launch_bf16_large<256>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+        if (tile == 128) return launch_bf16_large<128>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+    }
     if (big >= 512) {
         if (vec)
             launch_bf16_tile<S, SPLIT, 128, 128, 4>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, lower,

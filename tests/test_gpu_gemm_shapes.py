@@ -45,3 +45,13 @@ def test_split_k_lower_tiles_exact(lmx_gpu, n, k, trans):
     C = torch.zeros(n, n, dtype=torch.float64, device="cuda")
     lmx_gpu.syrk_dev(A, C, trans=trans)
     np.testing.assert_array_equal(C.cpu().numpy().astype(np.int64), va.T @ va if trans == "T" else va @ va.T)
+
+
+# BF16 tiles of 128 and 256 (at least 100 tiles of 128), remainders in m, n
+# and k; the last two shapes are not aligned for 16-byte vectors
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
+@pytest.mark.parametrize("m,n,k,pad", [(1288, 1304, 8, 0), (1288, 1280, 200, 8), (3080, 3000, 136, 0),
+                                       (3072, 3072, 64, 16), (1288, 1304, 72, 4), (1290, 1301, 67, 0)])
+def test_bf16_large_tiles_exact(lmx_gpu, m, n, k, pad, ta, tb):
+    import torch
+    check(torch, lmx_gpu.gemm_bf16_dev, torch.bfloat16, torch.float32, m, n, k, ta, tb, pad, 0, 3.0 if pad else 0.0)
