@@ -528,6 +528,11 @@ void potrs(hipStream_t s, int64_t n, int64_t nrhs, const T *L, int64_t lda, T *B
         tri_inverse_solve<T>(s, true, true, n, nrhs, L, lda, WU, B, ldb);
         return;
     }
+    if (tri_small_ok(n, nrhs)) {
+        const TriSolve sv[2] = {{true, false, false}, {true, true, false}};
+        tri_small<T>(s, n, nrhs, L, lda, nullptr, B, ldb, sv, 2);
+        return;
+    }
     trsm_left<T>(s, true, false, false, n, nrhs, L, lda, B, ldb);
     trsm_left<T>(s, true, true, false, n, nrhs, L, lda, B, ldb);
 }

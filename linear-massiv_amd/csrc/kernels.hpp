@@ -124,6 +124,17 @@ template <class T>
 void trsm_right(hipStream_t s, bool lower, bool trans, bool unit, int64_t nrows, int64_t n,
                 const T *A, int64_t lda, T *B, int64_t ldb);
 
+// Up to two triangular solves with the same stored matrix, one after the
+// other, in one launch: B <- op1(T1)^-1 op0(T0)^-1 P B, for sizes that
+// tri_small_ok takes; perm (may be null): row i of P B is row perm[i] of B.
+struct TriSolve {
+    bool lower, trans, unit;
+};
+bool tri_small_ok(int64_t n, int64_t nrhs);
+template <class T>
+void tri_small(hipStream_t s, int64_t n, int64_t nrhs, const T *A, int64_t lda, const int32_t *perm, T *B, int64_t ldb,
+               const TriSolve *sv, int solves);
+
 // Explicit inverses of the diagonal blocks of op(T) (blocks of order
 // tri_block(n), stored densely in tri_inverse_elems(n) elements of W), for
 // repeated solves with tri_inverse_solve (same lower / trans flags; B n x

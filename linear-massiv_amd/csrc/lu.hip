@@ -33,6 +33,7 @@
 // outer panel on the MFMA GEMM), then U12 = L11^{-1} A12 (TRSM through the
 // inverse of L11) and the trailing update A22 -= L21 U12 on the MFMA GEMM.
 #include <climits>
+#include <optional>
 #include <vector>
 
 #include "common.hpp"
@@ -1347,14 +1348,14 @@ __global__ __launch_bounds__(256) void row_gather_composed_kernel(T *__restrict_
     }
 }
 
-__global__ void iota_kernel(int32_t *p, int n) {
-    int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = i;
-}
-
-__global__ void zero_u32_kernel(unsigned *p, int n) {
-    int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < n) p[i] = 0u;
+// Start of a factorisation: info = 0, the first nsync words of the exchange
+// records cleared, perm (may be null) the identity.
+__global__ void getrf_init_kernel(unsigned *__restrict__ sync, int nsync, int32_t *__restrict__ perm, int n,
+                                  int32_t *__restrict__ info) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < nsync) sync[i] = 0u;
+    if (perm != nullptr && i < n) perm[i] = i;
+    if (i == 0) *info = 0;
 }
 
 __global__ void finish_kernel(const unsigned *err, int32_t *info) {
@@ -1535,8 +1536,10 @@ void getrf_impl(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_ipiv, in
     if (tournament && sizeof(T) != 4) fail_arg("getrf: tournament pivoting is for the FP32 factor");
     if (tournament && tie_last) fail_arg("getrf: the tie rule of lu needs column-by-column pivoting");
     if (bf16 && sizeof(T) != 4) fail_arg("getrf: BF16 updates are for the FP32-stored factor");
-    clear_info(s, d_info);
-    if (n == 0) return;
+    if (n == 0) {
+        clear_info(s, d_info);
+        return;
+    }
     TimedRegion trall("getrf", s, 2.0 / 3.0 * (double)n * (double)n * (double)n);
     const int N = (int)n;
     size_t sync_bytes = (sizeof(PanelSync<T>) + 255) & ~size_t(255);
@@ -1555,13 +1558,13 @@ void getrf_impl(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_ipiv, in
     T *Wall = reinterpret_cast<T *>(cur + stash_bytes);
     int32_t *pairs_all = reinterpret_cast<int32_t *>(cur + stash_bytes + inv_bytes);
     auto *ts = tournament ? reinterpret_cast<TsluScratch<T> *>(cur + stash_bytes + inv_bytes + pair_bytes) : nullptr;
-    hipLaunchKernelGGL(zero_u32_kernel, dim3((unsigned)cdiv(sync_clear_words<T>(), 256)), dim3(256), 0, s,
-                       (unsigned *)sy, sync_clear_words<T>());
+    // the exchange records are zeroed where panels of several workgroups use
+    // them (and a time-out of theirs is looked for at the end)
+    const bool exchanges = N > PANEL_ROWS;
+    const int nsync = exchanges ? sync_clear_words<T>() : 0;
+    hipLaunchKernelGGL(getrf_init_kernel, dim3((unsigned)cdiv(std::max(N, nsync), 256)), dim3(256), 0, s,
+                       (unsigned *)sy, nsync, d_perm, N, d_info);
     LMX_LAUNCH_CHECK();
-    if (d_perm) {
-        hipLaunchKernelGGL(iota_kernel, dim3((unsigned)cdiv(N, 256)), dim3(256), 0, s, d_perm, N);
-        LMX_LAUNCH_CHECK();
-    }
     // Lookahead: the caller's stream factors outer panel b + 1 while an
     // auxiliary stream applies panel b's update to the columns beyond
     // b + 1.  Row interchanges of a panel reach, on the caller's stream, its
@@ -1572,9 +1575,13 @@ void getrf_impl(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_ipiv, in
     //               record E(b); U12 and A22 -= L21 U12 on panel b+1's columns
     //   stream aux: wait E(b); swaps(b) on [0, k0); U12 and A22 -= L21 U12 on
     //               the columns beyond panel b+1; record F(b)
-    AuxStream la;
-    hipStream_t aux = la.aux;
-    hipEvent_t evE = la.ready, evF = la.done;
+    // With at most two outer panels nothing runs beyond the next one, and the
+    // events would only cost (20 us of n = 500's 1440).
+    const bool ahead = N > 2 * NB_OUTER;
+    std::optional<AuxStream> la;
+    if (ahead) la.emplace();
+    hipStream_t aux = ahead ? la->aux : s;
+    hipEvent_t evE = ahead ? la->ready : nullptr, evF = ahead ? la->done : nullptr;
     bool pending = false;  // evF marks the auxiliary stream's last block
     unsigned base = 0;
     for (int b = 0, k0 = 0; k0 < N; ++b, k0 += NB_OUTER) {
@@ -1641,8 +1648,10 @@ void getrf_impl(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_ipiv, in
         // other columns: E goes before those, so that no event marker sits
         // between them and the next panel.
         if (trail > 0) gather_rows_deferred<T>(s, A, lda, k0 + nbw, N, k0, N, pairs, np, true);
-        LMX_HIP(hipEventRecord(evE, s));
-        LMX_HIP(hipStreamWaitEvent(aux, evE, 0));
+        if (ahead) {
+            LMX_HIP(hipEventRecord(evE, s));
+            LMX_HIP(hipStreamWaitEvent(aux, evE, 0));
+        }
         if (trail > 0) {
             tri_inverse_solve<T>(s, true, false, nbw, narrow, A11, lda, W, A12, lda);
             trailing_update<T>(s, bf16, trail, narrow, nbw, A11 + (int64_t)nbw * lda, lda, A12,
@@ -1656,12 +1665,16 @@ void getrf_impl(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_ipiv, in
             trailing_update<T>(aux, bf16, trail, trail - narrow, nbw, A11 + (int64_t)nbw * lda, lda, A12 + narrow,
                                A12 + (int64_t)nbw * lda + narrow, true);
         }
-        LMX_HIP(hipEventRecord(evF, aux));
-        pending = true;
+        if (ahead) {
+            LMX_HIP(hipEventRecord(evF, aux));
+            pending = true;
+        }
     }
     if (pending) LMX_HIP(hipStreamWaitEvent(s, evF, 0));
-    hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(64), 0, s, &sy->error, d_info);
-    LMX_LAUNCH_CHECK();
+    if (exchanges) {
+        hipLaunchKernelGGL(finish_kernel, dim3(1), dim3(64), 0, s, &sy->error, d_info);
+        LMX_LAUNCH_CHECK();
+    }
 }
 
 template <class T>
@@ -1675,6 +1688,11 @@ void getrs_perm(hipStream_t s, int64_t n, int64_t nrhs, const T *LU, int64_t lda
                 int64_t ldb, const T *WL, const T *WU) {
     if (n == 0 || nrhs == 0) return;
     TimedRegion tr("getrs", s);
+    if (!(WL && WU) && tri_small_ok(n, nrhs)) {
+        const TriSolve sv[2] = {{true, false, true}, {false, false, false}};
+        tri_small<T>(s, n, nrhs, LU, lda, d_perm, B, ldb, sv, 2);
+        return;
+    }
     Scratch tmp((size_t)(n * nrhs) * sizeof(T), s);
     unsigned g = (unsigned)cdiv(n * nrhs, 256);
     hipLaunchKernelGGL(row_permute_kernel<T>, dim3(g), dim3(256), 0, s, B, ldb, tmp.as<T>(), nrhs, d_perm,

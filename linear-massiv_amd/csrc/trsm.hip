@@ -284,6 +284,182 @@ __global__ void copy_rows_kernel(const T *__restrict__ in, int64_t ldi, T *__res
     out[i * ldo + c] = in[i * ldi + c];
 }
 
+// ---------------------------------------------------------------- small orders
+//
+// M x = b for up to SMALL_MAX_N unknowns and SMALL_MAX_NRHS right-hand sides
+// in one workgroup, and up to two solves one after the other (L then U, or L
+// then L^T) in one launch.  A solve of this size is latency: through block
+// inverses the two solves of an LU at n = 100 were 15 launches and two 64 x 64
+// inverses of 30 us each, 106 us in all, here 16 us.
+//   Per 64-row block in dependency order: all waves stage the diagonal block
+// in LDS (coalesced; an upper block reversed, J M J is lower) and sum the
+// products with what is solved (eight lanes a row, or, for a transposed
+// operand, a lane a row and the waves over the columns), then wave 0 solves
+// the block: lane i holds x_i, step k broadcasts x_k by v_readlane.  Rows are
+// scaled by their diagonal element's reciprocal first (the right-hand side
+// with the last correction of a division), which leaves one readlane and one
+// FMA on the chain from unknown to unknown; where an element of the block's
+// diagonal is so small or large that the reciprocal would leave the range,
+// every unknown is divided instead.
+constexpr int SMALL_MAX_N = 768, SMALL_MAX_NRHS = 4, SMALL_T = 512;
+struct SmallSolve {
+    int mt, mlower, unit;
+};
+
+template <class T, int NR>
+__device__ __forceinline__ void small_block_solve(const T (*S)[TB + 1], T (&x)[NR], bool unit) {
+    const int lane = threadIdx.x & 63;
+    T res[NR];  // lane k's unknown once it is known: later steps leave x[k] behind
+    const T d = S[lane][lane], ad = fabs(d);
+    const T small = sizeof(T) == 8 ? T(1e-150) : T(1e-18), large = T(1) / small;
+    if (unit || __all(ad >= small && ad <= large)) {
+        const T r = unit ? T(1) : T(1) / d;
+#pragma unroll
+        for (int q = 0; q < NR; ++q) {
+            const T y0 = x[q] * r, y1 = fma(fma(-y0, d, x[q]), r, y0);
+            x[q] = unit ? x[q] : (isfinite(y1) ? y1 : y0);
+            res[q] = x[q];
+        }
+#pragma unroll 16
+        for (int k = 0; k < TB; ++k) {
+            const T l = S[lane][k] * r;
+#pragma unroll
+            for (int q = 0; q < NR; ++q) {
+                const T xk = bcast_lane(x[q], k);
+                res[q] = k == lane ? x[q] : res[q];
+                x[q] = fma(-l, xk, x[q]);
+            }
+        }
+    } else {
+        for (int k = 0; k < TB; ++k) {
+            const T l = S[lane][k];
+#pragma unroll
+            for (int q = 0; q < NR; ++q) {
+                const T y = x[q] / d, xk = bcast_lane(y, k);
+                res[q] = k == lane ? y : res[q];
+                x[q] = fma(-l, xk, x[q]);
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < NR; ++q) x[q] = res[q];
+}
+
+template <class T, int NR>
+__global__ __launch_bounds__(SMALL_T) void tri_small_kernel(int n, int nrhs, const T *__restrict__ A, int64_t lda,
+                                                            const int32_t *__restrict__ perm, T *__restrict__ B,
+                                                            int64_t ldb, SmallSolve s0, SmallSolve s1, int solves) {
+    __shared__ T S[TB][TB + 1];
+    __shared__ __attribute__((aligned(16))) T xs[SMALL_MAX_N][NR];
+    __shared__ T part[SMALL_T / 64][NR][TB];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    constexpr int NW = SMALL_T / 64;
+    for (int i = t; i < n; i += SMALL_T) {
+        const int64_t r = perm ? perm[i] : i;
+#pragma unroll
+        for (int q = 0; q < NR; ++q) xs[i][q] = q < nrhs ? B[r * ldb + q] : T(0);
+    }
+    const int nb = (n + TB - 1) / TB;
+    for (int sv = 0; sv < solves; ++sv) {
+        const SmallSolve m = sv == 0 ? s0 : s1;
+        for (int bi = 0; bi < nb; ++bi) {
+            const int r0 = (m.mlower ? bi : nb - 1 - bi) * TB, cnt = min(TB, n - r0);
+            // the diagonal block of M as a lower triangle, identity beyond it
+            T a[TB * TB / SMALL_T];
+#pragma unroll
+            for (int i = 0; i < TB * TB / SMALL_T; ++i) {
+                const int e = i * SMALL_T + t;
+                a[i] = A[(int64_t)(r0 + min(e >> 6, cnt - 1)) * lda + r0 + min(e & 63, cnt - 1)];
+            }
+            // products with the solved unknowns [c0, c1)
+            const int c0 = m.mlower ? 0 : r0 + cnt, c1 = m.mlower ? r0 : n;
+            __syncthreads();  // xs of the previous block, S free
+#pragma unroll
+            for (int i = 0; i < TB * TB / SMALL_T; ++i) {
+                const int e = i * SMALL_T + t, p = e >> 6, c = e & 63;  // stored row and column
+                int r = m.mt ? c : p, k = m.mt ? p : c;                // row and column of M
+                const bool in = r < cnt && k < cnt;
+                if (!m.mlower) {
+                    r = TB - 1 - r;
+                    k = TB - 1 - k;
+                }
+                S[r][k] = in ? (r == k && m.unit ? T(1) : a[i]) : (r == k ? T(1) : T(0));
+            }
+            T acc[NR];
+#pragma unroll
+            for (int q = 0; q < NR; ++q) acc[q] = T(0);
+            if (!m.mt) {
+                const int r = r0 + min(wave * 8 + lane / 8, cnt - 1);
+                const T *row = A + (int64_t)r * lda;
+                int c = c0 + lane % 8;
+                for (; c + 15 * 8 < c1; c += 16 * 8) {
+                    T v[16];
+#pragma unroll
+                    for (int u = 0; u < 16; ++u) v[u] = row[c + 8 * u];
+#pragma unroll
+                    for (int u = 0; u < 16; ++u)
+#pragma unroll
+                        for (int q = 0; q < NR; ++q) acc[q] = fma(v[u], xs[c + 8 * u][q], acc[q]);
+                }
+                for (; c < c1; c += 8) {
+                    const T v = row[c];
+#pragma unroll
+                    for (int q = 0; q < NR; ++q) acc[q] = fma(v, xs[c][q], acc[q]);
+                }
+#pragma unroll
+                for (int q = 0; q < NR; ++q) {
+                    T v = acc[q];
+                    v += dpp_f<0xB1, 0xF>(v);   // quad_perm 1,0,3,2
+                    v += dpp_f<0x4E, 0xF>(v);   // quad_perm 2,3,0,1
+                    v += dpp_f<0x141, 0xF>(v);  // row_half_mirror
+                    if (lane % 8 == 0) part[0][q][wave * 8 + lane / 8] = v;
+                }
+            } else {
+                const T *col = A + r0 + min(lane, cnt - 1);
+                int c = c0 + wave;
+                for (; c + 7 * NW < c1; c += 8 * NW) {
+                    T v[8];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u) v[u] = col[(int64_t)(c + NW * u) * lda];
+#pragma unroll
+                    for (int u = 0; u < 8; ++u)
+#pragma unroll
+                        for (int q = 0; q < NR; ++q) acc[q] = fma(v[u], xs[c + NW * u][q], acc[q]);
+                }
+                for (; c < c1; c += NW) {
+                    const T v = col[(int64_t)c * lda];
+#pragma unroll
+                    for (int q = 0; q < NR; ++q) acc[q] = fma(v, xs[c][q], acc[q]);
+                }
+#pragma unroll
+                for (int q = 0; q < NR; ++q) part[wave][q][lane] = acc[q];
+            }
+            __syncthreads();
+            if (wave == 0) {
+                // lane i: row i of the lower triangle
+                const int r = m.mlower ? lane : TB - 1 - lane;
+                T x[NR];
+#pragma unroll
+                for (int q = 0; q < NR; ++q) {
+                    T sum = part[0][q][r];
+                    if (m.mt)
+                        for (int w = 1; w < NW; ++w) sum += part[w][q][r];
+                    x[q] = r < cnt ? xs[r0 + r][q] - sum : T(0);
+                }
+                small_block_solve<T, NR>(S, x, m.unit != 0);
+#pragma unroll
+                for (int q = 0; q < NR; ++q)
+                    if (r < cnt) xs[r0 + r][q] = x[q];
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = t; i < n; i += SMALL_T)
+#pragma unroll
+        for (int q = 0; q < NR; ++q)
+            if (q < nrhs) B[(int64_t)i * ldb + q] = xs[i][q];
+}
+
 // ---------------------------------------------------------------- dispatch
 
 template <class T>
@@ -354,6 +530,36 @@ void leaf(hipStream_t s, bool mt, bool mlower, bool unit, int bs, int64_t nvec, 
 }
 
 }  // namespace
+
+// Where one workgroup is faster than the block-inverse launches (FP64, one
+// triangle, 1 / 4 right-hand sides: n = 100 14 / 15 against 47 / 48 us, 500
+// 40 / 61 against 66 / 68, 700 61 / 89 against 101 / 104, 1000 115 / 157
+// against 103 / 107: by then it is bound by one CU's reads of the triangle).
+bool tri_small_ok(int64_t n, int64_t nrhs) { return n <= SMALL_MAX_N && nrhs <= SMALL_MAX_NRHS; }
+
+template <class T>
+void tri_small(hipStream_t s, int64_t n, int64_t nrhs, const T *A, int64_t lda, const int32_t *perm, T *B, int64_t ldb,
+               const TriSolve *sv, int solves) {
+    if (n <= 0 || nrhs <= 0) return;
+    TimedRegion tr("trsm", s, (double)solves * (double)n * (double)n * (double)nrhs);
+    SmallSolve m[2] = {{0, 0, 0}, {0, 0, 0}};
+    for (int i = 0; i < solves; ++i) m[i] = {sv[i].trans, sv[i].lower != sv[i].trans, sv[i].unit};
+#define LMX_SMALL(NR_)                                                                                           \
+    hipLaunchKernelGGL((tri_small_kernel<T, NR_>), dim3(1), dim3(SMALL_T), 0, s, (int)n, (int)nrhs, A, lda, perm, B, \
+                       ldb, m[0], m[1], solves)
+    if (nrhs == 1)
+        LMX_SMALL(1);
+    else if (nrhs == 2)
+        LMX_SMALL(2);
+    else
+        LMX_SMALL(4);
+#undef LMX_SMALL
+    LMX_LAUNCH_CHECK();
+}
+template void tri_small<double>(hipStream_t, int64_t, int64_t, const double *, int64_t, const int32_t *, double *,
+                                int64_t, const TriSolve *, int);
+template void tri_small<float>(hipStream_t, int64_t, int64_t, const float *, int64_t, const int32_t *, float *, int64_t,
+                               const TriSolve *, int);
 
 int tri_block(int64_t n) {
     int b = TB;
@@ -435,6 +641,11 @@ void trsm_left(hipStream_t s, bool lower, bool trans, bool unit, int64_t n, int6
     if (n <= 0 || nrhs <= 0) return;
     if (n > INT32_MAX / 2 || nrhs > INT32_MAX / 2) fail_arg("trsm: dimension too large");
     TimedRegion tr("trsm", s, (double)n * (double)n * (double)nrhs);
+    if (tri_small_ok(n, nrhs)) {
+        const TriSolve sv{lower, trans, unit};
+        tri_small<T>(s, n, nrhs, A, lda, nullptr, B, ldb, &sv, 1);
+        return;
+    }
     if (n <= TB) {
         leaf<T, false>(s, trans, lower != trans, unit, (int)n, nrhs, A, lda, B, ldb);
         return;
