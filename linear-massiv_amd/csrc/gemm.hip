@@ -651,6 +651,134 @@ __global__ __launch_bounds__(64 * KS_WAVES) void gemm_ksplit_kernel(int m, int n
     }
 }
 
+// C = alpha op(A) op(B) + beta C, every wave for itself: no LDS, no barrier.
+// A wave owns a 16 MT x 16 NT tile (the workgroup 2 x 2 of them, which share
+// what they read in L1) and loads its MFMA operands from global memory two
+// 16-k chunks ahead, as gemm_ksplit_kernel does.
+//   An FP64 MFMA takes 64 cycles, so even 24 operand bytes a clock and CU leave
+// L1 and L2 time to spare, and the waves never wait for each other; the tiles
+// through LDS lost a quarter of the matrix cores' time to the barrier a step.
+// Operands as stored, a k-contiguous A costs 16 lines a load and B two, so the
+// tile is wide (64 x 128: 67 TF at 8192^3, 128 x 64: 60 TF).  No operand needs
+// to be aligned.  FP64 8192^3 20.8 -> 16.4 ms (52.9 -> 67.0 TF), A transposed
+// 24.7 -> 15.7 ms, 1999 x 1001 x 777 with A transposed 90 -> 62 us, 3001 x 2999
+// x 1003 588 -> 351 us.
+template <class T, int MT, int NT, bool TA, bool TB, bool VEC>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_direct_kernel(
+    int m, int n, int k, T alpha, const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb, T beta,
+    T *__restrict__ C, int64_t ldc, int tiles_m, int tiles_n) {
+    typedef typename Acc<T>::type V;
+    constexpr int ST = 2;  // chunks in flight
+    int tm, tn;
+    tile_of(tiles_m, tiles_n, false, tm, tn);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int m0 = (2 * tm + (wave >> 1)) * 16 * MT, n0 = (2 * tn + (wave & 1)) * 16 * NT;
+    const int lr = lane & 15, lk = lane >> 4;
+    struct Frag {
+        T a[MT][4], b[NT][4];
+    };
+    const T *pa[MT], *pb[NT];
+#pragma unroll
+    for (int a = 0; a < MT; ++a) {
+        const int64_t i = min(m0 + a * 16 + lr, m - 1);
+        pa[a] = TA ? A + i + (int64_t)(4 * lk) * lda : A + i * lda + 4 * lk;
+    }
+#pragma unroll
+    for (int b = 0; b < NT; ++b) {
+        const int64_t j = min(n0 + b * 16 + lr, n - 1);
+        pb[b] = TB ? B + j * ldb + 4 * lk : B + j + (int64_t)(4 * lk) * ldb;
+    }
+    auto operand = [&](const T *p, int64_t ld, bool along, T(&f)[4]) {
+        if (!along) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) f[s] = p[s * ld];
+        } else if constexpr (VEC) {
+            constexpr int E = V16<T>::N;
+#pragma unroll
+            for (int v = 0; v < 4 / E; ++v) {
+                const typename V16<T>::type x = *reinterpret_cast<const typename V16<T>::type *>(p + v * E);
+#pragma unroll
+                for (int q = 0; q < E; ++q) f[v * E + q] = x[q];
+            }
+        } else {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) f[s] = p[s];
+        }
+    };
+    auto load = [&](Frag &f, int64_t chunk) {
+        const int64_t oa = TA ? chunk * 16 * lda : chunk * 16, ob = TB ? chunk * 16 : chunk * 16 * ldb;
+#pragma unroll
+        for (int a = 0; a < MT; ++a) operand(pa[a] + oa, lda, !TA, f.a[a]);
+#pragma unroll
+        for (int b = 0; b < NT; ++b) operand(pb[b] + ob, ldb, TB, f.b[b]);
+    };
+    V acc[MT][NT];
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < NT; ++b) acc[a][b] = V{0, 0, 0, 0};
+    auto products = [&](const Frag &f) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int a = 0; a < MT; ++a)
+#pragma unroll
+                for (int b = 0; b < NT; ++b) acc[a][b] = mfma16x16x4(f.a[a][s], f.b[b][s], acc[a][b]);
+    };
+    const int full = k / 16;
+    if (full > 0) {
+        Frag f[ST];
+#pragma unroll
+        for (int u = 0; u < ST; ++u) load(f[u], min(u, full - 1));
+        int i = 0;
+        for (; i + ST <= full; i += ST)
+#pragma unroll
+            for (int u = 0; u < ST; ++u) {
+                products(f[u]);
+                load(f[u], min(i + u + ST, full - 1));
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+        for (int u = 0; u < ST - 1; ++u)
+            if (u < full - i) products(f[u]);
+    }
+    if ((k & 15) != 0) {
+        Frag f;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int64_t kk = (int64_t)full * 16 + 4 * lk + s, kc = (kk < k ? kk : k - 1) - 4 * lk;
+#pragma unroll
+            for (int a = 0; a < MT; ++a) {
+                const T x = TA ? pa[a][kc * lda] : pa[a][kc];
+                f.a[a][s] = kk < k ? x : T(0);
+            }
+#pragma unroll
+            for (int b = 0; b < NT; ++b) {
+                const T x = TB ? pb[b][kc] : pb[b][kc * ldb];
+                f.b[b][s] = kk < k ? x : T(0);
+            }
+        }
+        products(f);
+    }
+#pragma unroll
+    for (int a = 0; a < MT; ++a)
+#pragma unroll
+        for (int b = 0; b < NT; ++b) {
+            const int gj = n0 + b * 16 + lr;
+            if (gj >= n) continue;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int gi = m0 + a * 16 + acc_row<T>(lk, r);
+                if (gi < m) {
+                    T *c = C + (int64_t)gi * ldc + gj;
+                    T v = alpha * acc[a][b][r];
+                    if (beta != T(0)) v += beta * *c;
+                    *c = v;
+                }
+            }
+        }
+}
+
 // ---------------------------------------------------------------- BF16 tiles
 //
 // C (FP32) = alpha op(A) op(B) + beta C on v_mfma_f32_16x16x32_bf16 (FP32
@@ -1253,6 +1381,44 @@ int table_tile(int bytes, int64_t m, int64_t n, int64_t k) {
     return TILE_DEFAULT;
 }
 
+// gemm_direct_kernel where it beats the tiles through LDS: FP64, except
+// A B^T with aligned rows (51.7 TF through LDS, 49.9 TF direct at 4096^3: both
+// operands cost 16 lines a load; FP32, whose MFMA takes half the time for half
+// the bytes, lost everywhere), and enough tiles for the CUs (144 tiles, 1100 x
+// 1000 x 900: 69 against 87 us; 128 tiles, 1024^3: 75 against 67 us).  Returns
+// whether it took the product.
+constexpr int64_t DIRECT_FILL = 140;
+constexpr int DIRECT_MIN_K = 64;
+bool gemm_direct(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k, double alpha, const double *A,
+                 int64_t lda, const double *B, int64_t ldb, double beta, double *C, int64_t ldc) {
+    constexpr int MT = 2, NT = 4;
+    const BatchStrides nob{1, 0, 0, 0, 0, 0, 0};
+    if (tb && nn_ok<double>(ta, tb, n, k, A, lda, B, ldb, nob)) return false;
+    const int tiles_m = (int)cdiv(m, 32 * MT), tiles_n = (int)cdiv(n, 32 * NT);
+    if (k < DIRECT_MIN_K || (int64_t)tiles_m * tiles_n < DIRECT_FILL) return false;
+    auto al = [](const void *p, int64_t ld) { return ((uintptr_t)p & 15) == 0 && ld % 2 == 0; };
+    const bool vec = (ta || al(A, lda)) && (!tb || al(B, ldb));
+    TimedRegion tr("gemm", s, 2.0 * (double)m * (double)n * (double)k);
+#define LMX_DIRECT(TA_, TB_, VEC_)                                                                                   \
+    hipLaunchKernelGGL((gemm_direct_kernel<double, MT, NT, TA_, TB_, VEC_>), dim3(tiles_m *tiles_n), dim3(256), 0, s, \
+                       (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C, ldc, tiles_m, tiles_n)
+    if (ta && !tb)
+        LMX_DIRECT(true, false, true);  // no operand's k runs along memory
+    else if (!ta && !tb && vec)
+        LMX_DIRECT(false, false, true);
+    else if (!ta && !tb)
+        LMX_DIRECT(false, false, false);
+    else if (!ta)
+        LMX_DIRECT(false, true, false);
+    else if (vec)
+        LMX_DIRECT(true, true, true);
+    else
+        LMX_DIRECT(true, true, false);
+#undef LMX_DIRECT
+    LMX_LAUNCH_CHECK();
+    return true;
+}
+
 template <class T>
 void gemm_impl(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k, T alpha,
                const T *A, int64_t lda, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, size_t lds_footprint = 0,
@@ -1264,6 +1430,13 @@ void gemm_impl(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k,
     // A GEMM sharing its CUs with the LU panels keeps its measured tile (the
     // table is timed on an idle device); the others take the tuned table's
     // tile where it has one.
+    if constexpr (sizeof(T) == 8) {
+        // beside the LU panels only where the product is the longer of the two
+        // (FP64 LU n = 16384 141 -> 128 ms; at n = 8192 36.0 against 36.2 ms)
+        if ((!sharing || m > 8192) && lds_footprint == 0 && t_tile_override == TILE_DEFAULT &&
+            gemm_direct(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc))
+            return;
+    }
     const int tile = sharing ? TILE_DEFAULT : table_tile((int)sizeof(T), m, n, k);
     if (tile != TILE_DEFAULT) {
         const BatchStrides nob{1, 0, 0, 0, 0, 0, 0};

@@ -55,3 +55,13 @@ def test_split_k_lower_tiles_exact(lmx_gpu, n, k, trans):
 def test_bf16_large_tiles_exact(lmx_gpu, m, n, k, pad, ta, tb):
     import torch
     check(torch, lmx_gpu.gemm_bf16_dev, torch.bfloat16, torch.float32, m, n, k, ta, tb, pad, 0, 3.0 if pad else 0.0)
+
+
+# FP64 products on the wave-by-wave kernel (at least 140 tiles of 64 x 128):
+# k below, at and past one chunk's multiples, unaligned rows, ragged edges
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
+@pytest.mark.parametrize("m,n,k,pad,offset", [(1153, 1025, 64, 0, 0), (1100, 1030, 65, 1, 1), (640, 1800, 100, 0, 0),
+                                              (1999, 1001, 79, 2, 0), (1280, 1281, 96, 0, 1)])
+def test_fp64_direct_exact(lmx_gpu, m, n, k, pad, offset, ta, tb):
+    import torch
+    check(torch, lmx_gpu.dgemm_dev, torch.float64, torch.float64, m, n, k, ta, tb, pad, offset, 3.0 if pad else 0.0)
