@@ -524,8 +524,9 @@ void potrs(hipStream_t s, int64_t n, int64_t nrhs, const T *L, int64_t lda, T *B
            const T *WU) {
     if (n == 0 || nrhs == 0) return;
     if (WL && WU) {
-        tri_inverse_solve<T>(s, true, false, n, nrhs, L, lda, WL, B, ldb);
-        tri_inverse_solve<T>(s, true, true, n, nrhs, L, lda, WU, B, ldb);
+        Scratch mid((size_t)(n * nrhs) * sizeof(T), s);
+        tri_inverse_solve_to<T>(s, true, false, n, nrhs, L, lda, WL, B, ldb, mid.as<T>(), nrhs);
+        tri_inverse_solve_to<T>(s, true, true, n, nrhs, L, lda, WU, mid.as<T>(), nrhs, B, ldb);
         return;
     }
     if (tri_small_ok(n, nrhs)) {

@@ -126,6 +126,11 @@ RefineOut factor_solve(hipStream_t s, const lmx_factor_s *h, int64_t k, const do
         return out;
     }
     if (h->precision == LMX_PREC_F64) {
+        if (h->kind == LMX_FACTOR_LU && h->WL) {
+            getrs_perm_to<double>(s, n, k, h->F, n, h->perm, dB, ldb, dX, ldx, h->WL, h->WU);
+            out.converged = true;
+            return out;
+        }
         copy_d(s, dB, ldb, dX, ldx, n, k);
         if (h->kind == LMX_FACTOR_CHOLESKY)
             potrs<double>(s, n, k, h->F, n, dX, ldx, h->WL, h->WU);

@@ -143,6 +143,10 @@ int tri_block(int64_t n);
 int64_t tri_inverse_elems(int64_t n);
 template <class T>
 void tri_inverse_build(hipStream_t s, bool lower, bool trans, bool unit, int64_t n, const T *A, int64_t lda, T *W);
+// tri_inverse_solve_to leaves the solution in X (not B) and B updated.
+template <class T>
+void tri_inverse_solve_to(hipStream_t s, bool lower, bool trans, int64_t n, int64_t nrhs, const T *A, int64_t lda,
+                          const T *W, T *B, int64_t ldb, T *X, int64_t ldx);
 template <class T>
 void tri_inverse_solve(hipStream_t s, bool lower, bool trans, int64_t n, int64_t nrhs, const T *A, int64_t lda,
                        const T *W, T *B, int64_t ldb);
@@ -166,6 +170,10 @@ void getrf_impl(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_ipiv, in
 template <class T>
 void getrs_perm(hipStream_t s, int64_t n, int64_t nrhs, const T *LU, int64_t lda,
                 const int32_t *d_perm, T *B, int64_t ldb, const T *WL = nullptr, const T *WU = nullptr);
+// The same from B into X (B is only read; X = B allowed).
+template <class T>
+void getrs_perm_to(hipStream_t s, int64_t n, int64_t nrhs, const T *LU, int64_t lda, const int32_t *d_perm,
+                   const T *B, int64_t ldb, T *X, int64_t ldx, const T *WL, const T *WU);
 // Solve with getrf's factors and swap list.
 template <class T>
 void getrs(hipStream_t s, int64_t n, int64_t nrhs, const T *LU, int64_t lda,

@@ -1682,32 +1682,56 @@ void getrf(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_ipiv, int32_t
     getrf_impl<T>(s, n, A, lda, d_ipiv, nullptr, d_info);
 }
 
+// Solve with a permutation vector and the inverses of the factors' diagonal
+// blocks: X <- U^{-1} L^{-1} P B.
+template <class T>
+void getrs_perm_to(hipStream_t s, int64_t n, int64_t nrhs, const T *LU, int64_t lda, const int32_t *d_perm,
+                   const T *B, int64_t ldb, T *X, int64_t ldx, const T *WL, const T *WU) {
+    if (n == 0 || nrhs == 0) return;
+    TimedRegion tr("getrs", s);
+    // P B -> tmp; L: tmp -> mid; U: mid -> X, each solve into the next one's
+    // operand
+    const int64_t elems = cdiv(n * nrhs, 32) * 32;  // keeps mid aligned
+    Scratch tmp((size_t)(2 * elems) * sizeof(T), s);
+    T *pb = tmp.as<T>(), *mid = pb + elems;
+    hipLaunchKernelGGL(row_permute_kernel<T>, dim3((unsigned)cdiv(n * nrhs, 256)), dim3(256), 0, s, B, ldb, pb, nrhs,
+                       d_perm, (int)n, (int)nrhs);
+    LMX_LAUNCH_CHECK();
+    tri_inverse_solve_to<T>(s, true, false, n, nrhs, LU, lda, WL, pb, nrhs, mid, nrhs);
+    tri_inverse_solve_to<T>(s, false, false, n, nrhs, LU, lda, WU, mid, nrhs, X, ldx);
+}
+
 // Solve with a permutation vector: B <- U^{-1} L^{-1} P B.
 template <class T>
 void getrs_perm(hipStream_t s, int64_t n, int64_t nrhs, const T *LU, int64_t lda, const int32_t *d_perm, T *B,
                 int64_t ldb, const T *WL, const T *WU) {
     if (n == 0 || nrhs == 0) return;
-    TimedRegion tr("getrs", s);
-    if (!(WL && WU) && tri_small_ok(n, nrhs)) {
+    if (WL && WU) return getrs_perm_to<T>(s, n, nrhs, LU, lda, d_perm, B, ldb, B, ldb, WL, WU);
+    if (tri_small_ok(n, nrhs)) {
+        TimedRegion tr("getrs", s);
         const TriSolve sv[2] = {{true, false, true}, {false, false, false}};
         tri_small<T>(s, n, nrhs, LU, lda, d_perm, B, ldb, sv, 2);
         return;
     }
-    Scratch tmp((size_t)(n * nrhs) * sizeof(T), s);
-    unsigned g = (unsigned)cdiv(n * nrhs, 256);
-    hipLaunchKernelGGL(row_permute_kernel<T>, dim3(g), dim3(256), 0, s, B, ldb, tmp.as<T>(), nrhs, d_perm,
-                       (int)n, (int)nrhs);
-    LMX_LAUNCH_CHECK();
-    hipLaunchKernelGGL(copy2d_kernel<T>, dim3(g), dim3(256), 0, s, tmp.as<T>(), nrhs, B, ldb, (int)n,
-                       (int)nrhs);
-    LMX_LAUNCH_CHECK();
-    if (WL && WU) {
-        tri_inverse_solve<T>(s, true, false, n, nrhs, LU, lda, WL, B, ldb);
-        tri_inverse_solve<T>(s, false, false, n, nrhs, LU, lda, WU, B, ldb);
+    if (n <= 64) {  // one block: substitution, no inverses
+        TimedRegion tr("getrs", s);
+        Scratch tmp((size_t)(n * nrhs) * sizeof(T), s);
+        const dim3 g((unsigned)cdiv(n * nrhs, 256));
+        hipLaunchKernelGGL(row_permute_kernel<T>, g, dim3(256), 0, s, B, ldb, tmp.as<T>(), nrhs, d_perm, (int)n,
+                           (int)nrhs);
+        LMX_LAUNCH_CHECK();
+        hipLaunchKernelGGL(copy2d_kernel<T>, g, dim3(256), 0, s, tmp.as<T>(), nrhs, B, ldb, (int)n, (int)nrhs);
+        LMX_LAUNCH_CHECK();
+        trsm_left<T>(s, true, false, true, n, nrhs, LU, lda, B, ldb);
+        trsm_left<T>(s, false, false, false, n, nrhs, LU, lda, B, ldb);
         return;
     }
-    trsm_left<T>(s, true, false, true, n, nrhs, LU, lda, B, ldb);
-    trsm_left<T>(s, false, false, false, n, nrhs, LU, lda, B, ldb);
+    const size_t welems = (size_t)tri_inverse_elems(n);
+    Scratch w(2 * welems * sizeof(T), s);
+    T *wl = w.as<T>(), *wu = wl + welems;
+    tri_inverse_build<T>(s, true, false, true, n, LU, lda, wl);
+    tri_inverse_build<T>(s, false, false, false, n, LU, lda, wu);
+    getrs_perm_to<T>(s, n, nrhs, LU, lda, d_perm, B, ldb, B, ldb, wl, wu);
 }
 
 template <class T>
@@ -1731,6 +1755,10 @@ template void getrs<double>(hipStream_t, int64_t, int64_t, const double *, int64
                             int64_t);
 template void getrs<float>(hipStream_t, int64_t, int64_t, const float *, int64_t, const int32_t *, float *,
                            int64_t);
+template void getrs_perm_to<double>(hipStream_t, int64_t, int64_t, const double *, int64_t, const int32_t *,
+                                    const double *, int64_t, double *, int64_t, const double *, const double *);
+template void getrs_perm_to<float>(hipStream_t, int64_t, int64_t, const float *, int64_t, const int32_t *,
+                                   const float *, int64_t, float *, int64_t, const float *, const float *);
 template void getrs_perm<double>(hipStream_t, int64_t, int64_t, const double *, int64_t, const int32_t *,
                                  double *, int64_t, const double *, const double *);
 template void getrs_perm<float>(hipStream_t, int64_t, int64_t, const float *, int64_t, const int32_t *, float *,

@@ -605,18 +605,17 @@ void tri_inverse_build(hipStream_t s, bool lower, bool trans, bool unit, int64_t
 
 // op(T) X = B with the inverses of tri_inverse_build: for each diagonal
 // block in dependency order, X_b = W_b B_b, then the rows still unsolved
-// take B_i -= M_ib X_b -- two launches per block, each a full-chip pass.
+// take B_i -= M_ib X_b -- two launches per block, each a full-chip pass.  B is
+// left updated, the solution goes to X (not B): a caller with two solves hands
+// the first one's X to the second and needs no copies between.
 template <class T>
-void tri_inverse_solve(hipStream_t s, bool lower, bool trans, int64_t n, int64_t nrhs, const T *A, int64_t lda,
-                       const T *W, T *B, int64_t ldb) {
+void tri_inverse_solve_to(hipStream_t s, bool lower, bool trans, int64_t n, int64_t nrhs, const T *A, int64_t lda,
+                          const T *W, T *B, int64_t ldb, T *X, int64_t ldx) {
     if (n <= 0 || nrhs <= 0) return;
     if (n > INT32_MAX / 2 || nrhs > INT32_MAX / 2) fail_arg("trsm: dimension too large");
     TimedRegion tr("trsm", s, (double)n * (double)n * (double)nrhs);
     const bool mt = trans, mlower = lower != trans;
     const int bw = tri_block(n), nbw = (int)cdiv(n, bw);
-    Scratch sX((size_t)n * nrhs * sizeof(T), s);
-    T *X = sX.as<T>();
-    const int64_t ldx = nrhs;
     for (int bi = 0; bi < nbw; ++bi) {
         const int b = mlower ? bi : nbw - 1 - bi;
         const int64_t j0 = (int64_t)b * bw, nj = std::min<int64_t>(bw, n - j0);
@@ -628,7 +627,17 @@ void tri_inverse_solve(hipStream_t s, bool lower, bool trans, int64_t n, int64_t
             apply_block<T>(s, ni, nj, nrhs, T(-1), Mb, lda, mt, X + j0 * ldx, ldx, true, B + i0 * ldb, ldb);
         }
     }
-    hipLaunchKernelGGL(copy_rows_kernel<T>, dim3((unsigned)cdiv(n * nrhs, 256)), dim3(256), 0, s, X, ldx, B, ldb, n,
+}
+
+// The same in place on B.
+template <class T>
+void tri_inverse_solve(hipStream_t s, bool lower, bool trans, int64_t n, int64_t nrhs, const T *A, int64_t lda,
+                       const T *W, T *B, int64_t ldb) {
+    if (n <= 0 || nrhs <= 0) return;
+    Scratch sX((size_t)n * nrhs * sizeof(T), s);
+    T *X = sX.as<T>();
+    tri_inverse_solve_to<T>(s, lower, trans, n, nrhs, A, lda, W, B, ldb, X, nrhs);
+    hipLaunchKernelGGL(copy_rows_kernel<T>, dim3((unsigned)cdiv(n * nrhs, 256)), dim3(256), 0, s, X, nrhs, B, ldb, n,
                        (int)nrhs);
     LMX_LAUNCH_CHECK();
 }
@@ -697,8 +706,12 @@ template void trsm_left<float>(hipStream_t, bool, bool, bool, int64_t, int64_t, 
                                int64_t);
 template void tri_inverse_build<double>(hipStream_t, bool, bool, bool, int64_t, const double *, int64_t, double *);
 template void tri_inverse_build<float>(hipStream_t, bool, bool, bool, int64_t, const float *, int64_t, float *);
+template void tri_inverse_solve_to<double>(hipStream_t, bool, bool, int64_t, int64_t, const double *, int64_t,
+                                       const double *, double *, int64_t, double *, int64_t);
 template void tri_inverse_solve<double>(hipStream_t, bool, bool, int64_t, int64_t, const double *, int64_t,
                                         const double *, double *, int64_t);
+template void tri_inverse_solve_to<float>(hipStream_t, bool, bool, int64_t, int64_t, const float *, int64_t,
+                                       const float *, float *, int64_t, float *, int64_t);
 template void tri_inverse_solve<float>(hipStream_t, bool, bool, int64_t, int64_t, const float *, int64_t,
                                        const float *, float *, int64_t);
 template void trsm_right<double>(hipStream_t, bool, bool, bool, int64_t, int64_t, const double *, int64_t, double *,
