@@ -396,10 +396,16 @@ __device__ __forceinline__ void panel_column(PanelRows<T> &st, PanelLds<T> &L, b
     panel_offer<T, U, TL>(st, L, j, m);
     __syncthreads();
     const T *prow = L.prow[par ^ 1];
+    // a quad of lanes reads all offers at once; the best is picked from
+    // registers, not read again
+    const int x = threadIdx.x & 3;
+    const T sv = L.slot_v[par][x], sn = L.slot_n[par][x], sl = L.slot_l[par][x];
+    const T c1 = prow[(C1 + SH) & (KB - 1)];
+    const int sp = L.slot_pos[par][x];
     const int bw = panel_best<T, TL>(L, par);  // row j is always offered
-    const int p = L.slot_pos[par][bw];
-    T val[2] = {L.slot_v[par][bw], L.slot_n[par][bw]};
-    if (update) val[1] = fma(-L.slot_l[par][bw], prow[(C1 + SH) & (KB - 1)], val[1]);
+    const int p = __builtin_amdgcn_readlane(sp, bw);
+    T val[2] = {bcast_lane(sv, bw), bcast_lane(sn, bw)};
+    if (update) val[1] = fma(-bcast_lane(sl, bw), c1, val[1]);
     if (j > 0) panel_update<T, U>(st, L, update, prow, j, j0);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -740,32 +746,31 @@ __attribute__((amdgpu_waves_per_eu(PanelShape<T>::MIN_WAVES_PER_SIMD))) void get
     //     columns are solved between, U12 = L11^{-1} B12 (unit lower,
     //     x_i -= l_ik x_k with k ascending for every i).
     const int nd = min(kb, m);
-    if (t < 64) {
-        const int pj = t < kb ? L.pivs[t] : -1;
-        bool keep = t < kb && pj >= kb;
+    // the list is the fifth wave's while the others store their rows
+    if (wave == (MULTI ? S::WAVES : 0)) {
+        const int pj = lane < kb ? L.pivs[lane] : -1;
+        bool keep = lane < kb && pj >= kb;
 #pragma unroll
         for (int x = 0; x < KB; ++x) {
             const int px = __builtin_amdgcn_readlane(pj, x);
-            keep = keep && !(x < t && px == pj);
+            keep = keep && !(x < lane && px == pj);
         }
         const unsigned long long mask = __ballot(keep);
         const int cnt = nd + __popcll(mask);
-        if (t < nd) L.mv_dst[t] = t;
-        if (keep) L.mv_dst[nd + __popcll(mask & ((1ull << t) - 1ull))] = pj;
-        if (t >= cnt) L.mv_dst[t] = 0;
+        if (lane < nd) L.mv_dst[lane] = lane;
+        if (keep) L.mv_dst[nd + __popcll(mask & ((1ull << lane) - 1ull))] = pj;
+        if (lane >= cnt) L.mv_dst[lane] = 0;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        int pos = L.mv_dst[t];
+        int pos = L.mv_dst[lane];
         for (int jj = kb - 1; jj >= 0; --jj) {
             const int p = __builtin_amdgcn_readlane(pj, jj);
             pos = pos == jj ? p : (pos == p ? jj : pos);
         }
-        L.mv_src[t] = t < cnt ? pos : 0;
-        if (t == 0) {
-            L.mv_cnt = cnt;
-            if (w == 0 && local_info != 0 && *info == 0) *info = local_info;
-        }
+        L.mv_src[lane] = lane < cnt ? pos : 0;
+        if (lane == 0) L.mv_cnt = cnt;
     }
+    if (w == 0 && t == 0 && local_info != 0 && *info == 0) *info = local_info;
     __syncthreads();
     const int cnt = L.mv_cnt, dst = L.mv_dst[lane], src = L.mv_src[lane];
     if (w == 0 && wave == 0) {
@@ -788,14 +793,14 @@ __attribute__((amdgpu_waves_per_eu(PanelShape<T>::MIN_WAVES_PER_SIMD))) void get
         T x[2 * KB];
 #pragma unroll
         for (int e = 0; e < 2 * KB; ++e)
-            if (e < KB || e < cnt) x[e] = col[(int64_t)__builtin_amdgcn_readlane(src, e) * gx.ldg];
+            x[e] = col[(int64_t)__builtin_amdgcn_readlane(src, e) * gx.ldg];  // past cnt: row 0, not used
         if (u12 && cc >= n1) {
 #pragma unroll
             for (int k = 0; k < KB - 1; ++k) {
 #pragma unroll
                 for (int i = k + 1; i < KB; ++i) x[i] = fma(-L.l11[k][i], x[k], x[i]);
                 // the next columns of L11 stay in LDS until their turn
-                if (k % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+                if (k % (sizeof(T) == 8 ? 2 : 4) == 1) __builtin_amdgcn_sched_barrier(0);
             }
         }
         if (c < ncols) {
