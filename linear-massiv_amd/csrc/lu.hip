@@ -1662,7 +1662,8 @@ void getrf_impl(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_ipiv, in
             trailing_update<T>(s, bf16, trail, narrow, nbw, A11 + (int64_t)nbw * lda, lda, A12,
                                A12 + (int64_t)nbw * lda, false);
         }
-        gather_rows_deferred<T>(aux, A, lda, 0, k0, k0, N, pairs, np, false);
+        // beside panels the kernel with the small LDS footprint
+        gather_rows_deferred<T>(aux, A, lda, 0, k0, k0, N, pairs, np, !ahead);
         if (trail > narrow) {
             tri_inverse_solve<T>(aux, true, false, nbw, trail - narrow, A11, lda, W, A12 + narrow, lda);
             // at most two GEMM workgroups per CU, so every CU keeps room for
