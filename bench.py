@@ -600,17 +600,17 @@ def main():
         cnt, ms, work = fam[dom]["launches"], fam[dom]["ms_per_step"], fam[dom]["work_per_step"]
         achieved = work / (ms * 1e-3) / 1e12
         roofline = {"bound": "mfma",
-                    # the FP64 GEMMs of these workloads take the NN kernel (no
-                    # transposes, aligned rows): 128 x 64 tiles for the plain
-                    # GEMM, 128 x 128 beside the LU panels; the FP32 trailing
-                    # GEMM of the mixed LU shares its CUs with the panels and
-                    # keeps the first kernel
-                    "kernel": {"gemm": "gemm_nn_kernel<double, 128, 64>" if wl == "gemm_fp64"
+                    # the plain FP64 GEMM takes the kernel without LDS; the
+                    # FP64 LU's updates (n = 8192) the NN kernel's 128 x 128
+                    # tiles beside its panels; the FP32 trailing GEMM of the
+                    # mixed LU shares its CUs with the panels and keeps the
+                    # general kernel
+                    "kernel": {"gemm": "gemm_direct_kernel (64 x 128)" if wl == "gemm_fp64"
                                else "gemm_nn_kernel<double, 128, 128>",
                                "sgemm": "gemm_mfma_kernel<float, 128, 128, 16>",
                                "syrk": "gemm_nn_kernel<double, B^T> (lower tiles)",
                                "ssyrk": "gemm_nn_kernel<float, B^T> (lower tiles)",
-                               "bgemm": "gemm_bf16_kernel<bf16, 128, 128>",
+                               "bgemm": "gemm_bf16_large_kernel<256>",
                                "bgemm3": "gemm_bf16_kernel<float, split, 128, 128> (3 BF16 MFMAs a product)"}[dom],
                     "achieved": round(achieved, 3), "peak": PEAK[dom], "unit": "TFLOP/s",
                     "frac": round(achieved / PEAK[dom], 4), "traffic": profiled_traffic(wl, n, dom),

@@ -7,8 +7,10 @@
 // step's global loads are issued into registers before the current step's
 // MFMAs and written to the other buffer after them, one barrier per step.
 //
-// The NN case (both operands as stored) with 16-byte aligned rows has its
-// own kernel, gemm_nn_kernel, described there.
+// Other kernels, each described where it is: gemm_nn_kernel (both operands
+// as stored, 16-byte aligned rows), gemm_direct_kernel (FP64, operands
+// loaded by the waves that use them, no LDS), gemm_ksplit_kernel (outputs
+// whose 64 x 64 tiles leave the chip idle), and the BF16 kernels.
 //
 // MFMA 16x16x4 operands (f64 and f32 alike): lane l supplies
 // A[i = l%16][kk = l/16] and B[kk = l/16][j = l%16], so both operand tiles
@@ -1460,10 +1462,12 @@ void gemm_impl(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k,
     if (big_tiles >= 512) {
         TimedRegion tr(sizeof(T) == 8 ? "gemm" : "sgemm", s, flops);
         const BatchStrides nob{1, 0, 0, 0, 0, 0, 0};
-        // FP64 NN: 128 x 64 tiles (224 registers a wave against 392 at
-        // 128 x 128, so two waves share a SIMD): dgemm 8192^3 46 -> 53 TF.  A
-        // GEMM beside the LU panels keeps 128 x 128: faster, it slowed the
-        // panels more (FP64 LU at n=8192: 75.2 against 72.4 ms).
+        // FP64 NN below gemm_direct's limits, and aligned A B^T: 128 x 64
+        // tiles (224 registers a wave against 392 at 128 x 128, so two waves
+        // share a SIMD): 46 -> 53 TF at 8192^3.  A GEMM beside the LU panels
+        // keeps 128 x 128 where gemm_direct leaves it (m <= 8192): with
+        // 128 x 64 the panels slowed more than the GEMM gained (FP64 LU at
+        // n=8192: 75.2 against 72.4 ms).
         if (sizeof(T) == 8 && !sharing && nn_ok<T>(ta, tb, n, k, A, lda, B, ldb, nob))
             launch_tile<T, 128, 64, 16>(s, ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C, ldc, 0, 1,
                                         nob, lds_footprint);

@@ -46,10 +46,10 @@ namespace lmx {
 namespace {
 
 constexpr int KB = 32;        // panel kernel width
-constexpr int RPT = 1;        // rows per thread in the panel kernel
-constexpr int PT = 512;       // threads per panel workgroup (8 waves)
-constexpr int PW = PT / 64;   // waves per panel workgroup
-constexpr int PANEL_ROWS = PT * RPT;
+constexpr int RPT = 1;        // rows per thread in the tournament kernels
+constexpr int PT = 512;       // their threads (8 waves)
+constexpr int PW = PT / 64;
+constexpr int PANEL_ROWS = PT * RPT;  // rows of a panel workgroup, here and in getf2_panel_kernel
 constexpr int MAXP = 64;      // max panel workgroups (panel height <= 32768)
 constexpr int NB_OUTER = 256; // outer panel width (k of the trailing GEMM)
 constexpr long SPIN_LIMIT = 1L << 22;
@@ -62,8 +62,8 @@ constexpr long SPIN_LIMIT = 1L << 22;
 // whole factorisation (the records are zeroed once per getrf) and records are
 // double-buffered by column parity.
 //   key record:  a workgroup's offer for column j (three numbers), in a
-//                64-byte line of its own (32 workgroups polling packed keys:
-//                0.96 us an exchange, keys a line apart: 0.73 us)
+//                64-byte line of its own (an exchange of 32 workgroups spread
+//                over the XCDs: packed keys 1.43 us, keys a line apart 1.08)
 //   row record:  the whole row it offers
 constexpr int POS_BITS = 16;
 constexpr int POS_NONE = (1 << POS_BITS) - 1;  // above every position of a panel
@@ -205,15 +205,6 @@ __device__ __forceinline__ void wg_select(const T *vals, const int *ids, T &best
         bid = take ? id[x] : bid;
         bw = take ? x : bw;
     }
-}
-
-// The tie rule's bit among the set bits of a wave-uniform mask whose bit
-// order is row order: the lowest (rawPivotSearch) or the highest (lu's
-// maximumBy); -1 for an empty mask.
-template <bool TL>
-__device__ __forceinline__ int tie_index(unsigned long long mask) {
-    if (mask == 0) return -1;
-    return TL ? 63 - __builtin_clzll(mask) : __builtin_ctzll(mask);
 }
 
 // |x| as a pair of integers ordered like it (hi, then lo); hi is 0 for a row

@@ -14,7 +14,9 @@
 //     inverse and one update of all unsolved rows -- every launch spans
 //     the chip, and the work is one read of the triangle.  A factor that is
 //     solved with many times keeps its inverses (tri_inverse_build once,
-//     tri_inverse_solve per solve).
+//     tri_inverse_solve per solve);
+//   - a small factor with few right-hand sides ("small"): tri_small_kernel,
+//     one workgroup, one launch for both triangles of a factor, no inverses.
 #include "common.hpp"
 #include "device.hpp"
 #include "kernels.hpp"
