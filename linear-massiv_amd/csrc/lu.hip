@@ -59,14 +59,24 @@ constexpr long SPIN_LIMIT = 1L << 22;
 // tag of the column it belongs to and the position of the row it offers,
 // written with one device-coherent store; a reader polls a word until its tag
 // matches, so the poll is the load and no flag is needed.  Tags grow over the
-// whole factorisation (the records are zeroed once per getrf) and records are
-// double-buffered by column parity.
+// whole factorisation (the records are zeroed once per getrf).
 //   key record:  a workgroup's offer for column j (three numbers), in a
 //                64-byte line of its own (an exchange of 32 workgroups spread
 //                over the XCDs: packed keys 1.43 us, keys a line apart 1.08)
 //   row record:  the whole row it offers
+// Buffers: a tag has to match exactly, so a record may be written again only
+// when every reader has had it.  A column has three barriers.
+//   Keys, two buffers: a workgroup reads the keys of column j before its third
+// barrier and publishes its own key j + 1 after it; key j + 2 is written by a
+// workgroup that has received every key j + 1.
+//   Rows, three: a workgroup v reads row j beside publishing key j + 1, before
+// its second barrier of column j + 1, so it is key j + 2 that says v has had
+// it.  Row j + 2 is stored by a workgroup that has received the keys j + 1
+// alone (two buffers would let it overtake a slow v, which then waits until
+// its time-out); row j + 3 by one that has received every key j + 2.
 constexpr int POS_BITS = 16;
 constexpr int POS_NONE = (1 << POS_BITS) - 1;  // above every position of a panel
+constexpr int ROW_BUFS = 3;
 template <class T>
 struct PanelRec {
     static constexpr int WPV = sizeof(T) / 4;
@@ -76,10 +86,11 @@ struct PanelRec {
 template <class T>
 struct PanelSync {
     unsigned long long key[2][MAXP][PanelRec<T>::KEYW];
-    unsigned long long row[2][MAXP][PanelRec<T>::ROWW];
+    unsigned long long row[ROW_BUFS][MAXP][PanelRec<T>::ROWW];
     unsigned error;
     unsigned pad[63];
 };
+__device__ inline int row_slot(int j) { return (int)((unsigned)j % ROW_BUFS); }
 template <class T>
 constexpr int sync_clear_words() {
     return (int)(sizeof(PanelSync<T>) / 4);
@@ -448,7 +459,7 @@ __device__ __forceinline__ void panel_receive_row(PanelLds<T> &L, PanelComm &cm,
     const int lane = threadIdx.x & 63;
     if (lane < ROWW) {
         unsigned long long v[1] = {cm.rw};
-        panel_await(sy->row[(j - 1) & 1][cm.src] + lane, v, base + (unsigned)j, sy, cm.failed);
+        panel_await(sy->row[row_slot(j - 1)][cm.src] + lane, v, base + (unsigned)j, sy, cm.failed);
         reinterpret_cast<unsigned *>(L.prow[0])[lane] = (unsigned)v[0];
     }
     cm.failed = __any(cm.failed);
@@ -493,7 +504,7 @@ __device__ __forceinline__ void panel_communicate(PanelLds<T> &L, int kb, int P,
             L.res[1] = v1;
         }
         cm.src = gl;
-        cm.rw = xload(sy->row[j & 1][gl] + min(lane, R::ROWW - 1));
+        cm.rw = xload(sy->row[row_slot(j)][gl] + min(lane, R::ROWW - 1));
         update = gw >= 0 && bcast_lane(v0, gl) != T(0);
         __syncthreads();
     }
@@ -541,7 +552,7 @@ __device__ __forceinline__ void panel_column_multi(PanelRows<T> &st, PanelLds<T>
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         if (lane < R::ROWW)
-            xstore(sy->row[par][w] + lane, tagword(reinterpret_cast<const unsigned *>(L.stage)[lane], tg));
+            xstore(sy->row[row_slot(j)][w] + lane, tagword(reinterpret_cast<const unsigned *>(L.stage)[lane], tg));
     }
     __syncthreads();
     const T val[2] = {L.res[0], L.res[1]};
