@@ -79,3 +79,46 @@ def test_infinities_and_nan_as_unblocked_elimination(lmx_gpu, special, row, col)
     np.testing.assert_array_equal(ipiv, piv)
     np.testing.assert_array_equal(np.isnan(LU), np.isnan(W))
     np.testing.assert_array_equal(np.isinf(LU), np.isinf(W))
+
+
+@pytest.mark.parametrize("special", [np.inf, np.nan])
+@pytest.mark.parametrize("n,row,col", [(545, 0, 3), (545, 540, 0), (1100, 5, 5), (1100, 700, 17), (1100, 1099, 31)])
+def test_special_values_over_several_workgroups(lmx_gpu, special, n, row, col):
+    # the first panel (32 columns, 512 rows a workgroup) against the unblocked
+    # elimination of the same columns, in the final order of the rows
+    A = np.random.default_rng(row + 40 * col).integers(-4, 5, (n, n)).astype(float)
+    A[row, col] = special
+    LU, ipiv, _ = lmx_gpu.getrf(A)
+    W = A[:, :32].copy()
+    with np.errstate(all="ignore"):
+        for j in range(32):
+            p = j
+            if not np.isnan(W[j, j]):
+                best = np.where(np.isnan(W[j:, j]), -1.0, np.abs(W[j:, j]))
+                p = j + int(np.argmax(best))  # the lowest row of the largest
+            assert ipiv[j] == p
+            W[[j, p]] = W[[p, j]]
+            if W[j, j] != 0:
+                W[j + 1:, j] /= W[j, j]
+                W[j + 1:, j + 1:] -= np.outer(W[j + 1:, j], W[j, j + 1:])
+    for j in range(32, n):
+        W[[j, ipiv[j]]] = W[[ipiv[j], j]]
+    np.testing.assert_array_equal(np.isnan(LU[:, :32]), np.isnan(W))
+    np.testing.assert_array_equal(np.isinf(LU[:, :32]), np.isinf(W))
+
+
+@pytest.mark.parametrize("pad", [1, 2])
+@pytest.mark.parametrize("n", [129, 545, 1025])
+def test_chained_pivots_with_row_strides(lmx_gpu, n, pad):
+    # rows that do not start on 16-byte boundaries, and a stride
+    import torch
+    A, L, U, perm = chained(n, "random")
+    buf = torch.full((n * (n + pad) + 1,), 7.0, dtype=torch.float64, device="cuda")
+    dA = buf[1:].view(n, n + pad)[:, :n]
+    dA.copy_(torch.tensor(A))
+    ipiv = torch.zeros(n, dtype=torch.int32, device="cuda")
+    info = torch.zeros(1, dtype=torch.int32, device="cuda")
+    lmx_gpu.getrf_dev(dA, ipiv, info)
+    np.testing.assert_array_equal(lmx_gpu.swaps_to_perm(ipiv.cpu().numpy()), perm)
+    np.testing.assert_array_equal(dA.cpu().numpy(), np.tril(L, -1) + U)
+    assert bool((buf[1:].view(n, n + pad)[:, n:] == 7.0).all())
