@@ -17,6 +17,8 @@
 //     tri_inverse_solve per solve);
 //   - a small factor with few right-hand sides ("small"): tri_small_kernel,
 //     one workgroup, one launch for both triangles of a factor, no inverses.
+#include <cfloat>
+
 #include "common.hpp"
 #include "device.hpp"
 #include "kernels.hpp"
@@ -300,47 +302,92 @@ __global__ void copy_rows_kernel(const T *__restrict__ in, int64_t ldi, T *__res
 // the block: lane i holds x_i, step k broadcasts x_k by v_readlane.  Rows are
 // scaled by their diagonal element's reciprocal first (the right-hand side
 // with the last correction of a division), which leaves one readlane and one
-// FMA on the chain from unknown to unknown; where an element of the block's
-// diagonal is so small or large that the reciprocal would leave the range,
-// every unknown is divided instead.
+// FMA on the chain from unknown to unknown.
+//   Scaling must not leave the range where the substitution does not.  A scaled
+// element or right-hand side that overflows makes its unknown infinite or NaN;
+// one that is lost below the smallest normal number is looked for by the other
+// waves while wave 0 solves (in the loop of 64 steps the comparisons took 2 us
+// a block).  Where either is found, before the next block, wave 0 solves the
+// block again with a division an unknown, as it does at once where an element
+// of the diagonal is so small or large that its reciprocal is no use.
 constexpr int SMALL_MAX_N = 768, SMALL_MAX_NRHS = 4, SMALL_T = 512;
 struct SmallSolve {
     int mt, mlower, unit;
 };
 
+template <class T>
+__device__ __forceinline__ bool below_normal(T x) {
+    return x != T(0) && fabs(x) < (sizeof(T) == 8 ? T(DBL_MIN) : T(FLT_MIN));
+}
+
+// Whether row `lane` has a reciprocal to scale it by.
+template <class T>
+__device__ __forceinline__ bool small_scales(const T (*S)[TB + 1]) {
+    const T ad = fabs(S[threadIdx.x & 63][threadIdx.x & 63]);
+    const T small = sizeof(T) == 8 ? T(1e-150) : T(1e-18), large = T(1) / small;
+    return ad >= small && ad <= large;
+}
+
+// Whether scaling loses one of the columns first, first + step, ... of row
+// `lane`.
+template <class T>
+__device__ __forceinline__ bool small_ratios_lost(const T (*S)[TB + 1], int first, int step) {
+    const int lane = threadIdx.x & 63;
+    const T r = T(1) / S[lane][lane];
+    bool lost = false;
+    for (int k = first; k < TB; k += step) {
+        const T e = S[lane][k], l = e * r;
+        lost = lost || (k < lane && e != T(0) && (l == T(0) || below_normal(l)));
+    }
+    return lost;
+}
+
+// The block's unknowns from scaled rows; returns whether one of this lane's
+// left the range on the way.
 template <class T, int NR>
-__device__ __forceinline__ void small_block_solve(const T (*S)[TB + 1], T (&x)[NR], bool unit) {
+__device__ __forceinline__ bool small_block_scaled(const T (*S)[TB + 1], T (&x)[NR], bool unit) {
     const int lane = threadIdx.x & 63;
     T res[NR];  // lane k's unknown once it is known: later steps leave x[k] behind
-    const T d = S[lane][lane], ad = fabs(d);
-    const T small = sizeof(T) == 8 ? T(1e-150) : T(1e-18), large = T(1) / small;
-    if (unit || __all(ad >= small && ad <= large)) {
-        const T r = unit ? T(1) : T(1) / d;
+    const T d = S[lane][lane], r = unit ? T(1) : T(1) / d;
+    bool lost = false;
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+        const T y0 = x[q] * r, y1 = fma(fma(-y0, d, x[q]), r, y0);
+        lost = lost || (x[q] != T(0) && (y0 == T(0) || below_normal(y0)));
+        x[q] = unit ? x[q] : (isfinite(y1) ? y1 : y0);
+        res[q] = x[q];
+    }
+#pragma unroll 16
+    for (int k = 0; k < TB; ++k) {
+        const T l = S[lane][k] * r;
 #pragma unroll
         for (int q = 0; q < NR; ++q) {
-            const T y0 = x[q] * r, y1 = fma(fma(-y0, d, x[q]), r, y0);
-            x[q] = unit ? x[q] : (isfinite(y1) ? y1 : y0);
-            res[q] = x[q];
+            const T xk = bcast_lane(x[q], k);
+            res[q] = k == lane ? x[q] : res[q];
+            x[q] = fma(-l, xk, x[q]);
         }
-#pragma unroll 16
-        for (int k = 0; k < TB; ++k) {
-            const T l = S[lane][k] * r;
+    }
 #pragma unroll
-            for (int q = 0; q < NR; ++q) {
-                const T xk = bcast_lane(x[q], k);
-                res[q] = k == lane ? x[q] : res[q];
-                x[q] = fma(-l, xk, x[q]);
-            }
-        }
-    } else {
-        for (int k = 0; k < TB; ++k) {
-            const T l = S[lane][k];
+    for (int q = 0; q < NR; ++q) {
+        x[q] = res[q];
+        lost = lost || !isfinite(x[q]) || below_normal(x[q]);
+    }
+    return lost && !unit;
+}
+
+// The same by substitution, a division an unknown.
+template <class T, int NR>
+__device__ __forceinline__ void small_block_divided(const T (*S)[TB + 1], T (&x)[NR]) {
+    const int lane = threadIdx.x & 63;
+    T res[NR];
+    const T d = S[lane][lane];
+    for (int k = 0; k < TB; ++k) {
+        const T l = S[lane][k];
 #pragma unroll
-            for (int q = 0; q < NR; ++q) {
-                const T y = x[q] / d, xk = bcast_lane(y, k);
-                res[q] = k == lane ? y : res[q];
-                x[q] = fma(-l, xk, x[q]);
-            }
+        for (int q = 0; q < NR; ++q) {
+            const T y = x[q] / d, xk = bcast_lane(y, k);
+            res[q] = k == lane ? y : res[q];
+            x[q] = fma(-l, xk, x[q]);
         }
     }
 #pragma unroll
@@ -354,8 +401,29 @@ __global__ __launch_bounds__(SMALL_T) void tri_small_kernel(int n, int nrhs, con
     __shared__ T S[TB][TB + 1];
     __shared__ __attribute__((aligned(16))) T xs[SMALL_MAX_N][NR];
     __shared__ T part[SMALL_T / 64][NR][TB];
+    __shared__ int lost[SMALL_T / 64];  // per wave: what it found out of range in the last block
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     constexpr int NW = SMALL_T / 64;
+    if (t < NW) lost[t] = 0;
+    // wave 0: the last block's right-hand side, and where its unknown belongs
+    // (-1: nowhere, or solved by division already)
+    T rhs[NR];
+    int at = -1;
+    // the last block is done: solved again where a wave found it out of range
+    auto settle = [&]() {
+        __syncthreads();
+        int any = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) any |= lost[w];
+        if (any == 0) return;
+        if (wave == 0) {
+            small_block_divided<T, NR>(S, rhs);
+#pragma unroll
+            for (int q = 0; q < NR; ++q)
+                if (at >= 0) xs[at][q] = rhs[q];
+        }
+        __syncthreads();
+    };
     for (int i = t; i < n; i += SMALL_T) {
         const int64_t r = perm ? perm[i] : i;
 #pragma unroll
@@ -375,7 +443,7 @@ __global__ __launch_bounds__(SMALL_T) void tri_small_kernel(int n, int nrhs, con
             }
             // products with the solved unknowns [c0, c1)
             const int c0 = m.mlower ? 0 : r0 + cnt, c1 = m.mlower ? r0 : n;
-            __syncthreads();  // xs of the previous block, S free
+            settle();  // xs of the previous block, S free
 #pragma unroll
             for (int i = 0; i < TB * TB / SMALL_T; ++i) {
                 const int e = i * SMALL_T + t, p = e >> 6, c = e & 63;  // stored row and column
@@ -448,14 +516,27 @@ __global__ __launch_bounds__(SMALL_T) void tri_small_kernel(int n, int nrhs, con
                         for (int w = 1; w < NW; ++w) sum += part[w][q][r];
                     x[q] = r < cnt ? xs[r0 + r][q] - sum : T(0);
                 }
-                small_block_solve<T, NR>(S, x, m.unit != 0);
+                const bool scaled = m.unit || __all(small_scales<T>(S));
+                at = scaled && r < cnt ? r0 + r : -1;
+#pragma unroll
+                for (int q = 0; q < NR; ++q) rhs[q] = x[q];
+                bool out = false;
+                if (scaled)
+                    out = small_block_scaled<T, NR>(S, x, m.unit != 0);
+                else
+                    small_block_divided<T, NR>(S, x);
+                out = __any(out);
 #pragma unroll
                 for (int q = 0; q < NR; ++q)
                     if (r < cnt) xs[r0 + r][q] = x[q];
+                if (lane == 0) lost[0] = out;
+            } else {
+                const bool out = __any(!m.unit && small_ratios_lost<T>(S, wave - 1, NW - 1));
+                if (lane == 0) lost[wave] = out;
             }
         }
     }
-    __syncthreads();
+    settle();
     for (int i = t; i < n; i += SMALL_T)
 #pragma unroll
         for (int q = 0; q < NR; ++q)
