@@ -90,7 +90,9 @@ __global__ __launch_bounds__(256) void norm_inf_rows_kernel(const double *__rest
 // COLMAX_ROWS rows and 64 columns (blockIdx.y), reduces in LDS, and issues
 // one atomic per column.  32 rows a workgroup: 8 loads a thread, all in
 // flight (1024 rows a workgroup left 4 of them for n = 4096, each thread
-// waiting for 256 loads: 67 us for 4096 x 64).
+// waiting for 256 loads: 67 us for 4096 x 64).  NaN becomes +inf first (as
+// the atomic would make it): a comparison that lets NaN through would let the
+// next element replace it.
 constexpr int COLMAX_ROWS = 32;
 __global__ __launch_bounds__(256) void colmax_kernel(const double *__restrict__ X, int64_t ldx, int64_t n,
                                                      int ncols, double *__restrict__ out) {
@@ -105,21 +107,17 @@ __global__ __launch_bounds__(256) void colmax_kernel(const double *__restrict__ 
         for (int u = 0; u < COLMAX_ROWS / 4; ++u) v[u] = fabs(X[min(r0 + q + 4 * u, n - 1) * ldx + c]);
 #pragma unroll
         for (int u = 0; u < COLMAX_ROWS / 4; ++u)
-            if (!(v[u] <= m)) m = v[u];  // keeps NaN; a row past the end repeats the last one
+            m = fmax(m, isnan(v[u]) ? __builtin_huge_val() : v[u]);  // a row past the end repeats the last one
     }
     part[q][cl] = m;
     __syncthreads();
-    if (q == 0 && c < ncols) {
-        double r = part[0][cl];
-        for (int x = 1; x < 4; ++x)
-            if (!(part[x][cl] <= r)) r = part[x][cl];
-        atomic_max_nonneg(&out[c], r);
-    }
+    if (q == 0 && c < ncols)
+        atomic_max_nonneg(&out[c], fmax(fmax(part[0][cl], part[1][cl]), fmax(part[2][cl], part[3][cl])));
 }
 
 // The same for at most 8 columns: one thread per row (16 rows per thread,
 // coalesced), wave and workgroup reductions, one atomic per column and
-// workgroup.  NaN becomes +inf first (as the atomic would make it).
+// workgroup.
 constexpr int COLMAX_FEW = 8;
 __global__ __launch_bounds__(256) void colmax_few_kernel(const double *__restrict__ X, int64_t ldx, int64_t n,
                                                          int ncols, double *__restrict__ out) {

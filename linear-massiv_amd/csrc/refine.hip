@@ -46,7 +46,7 @@ __global__ void eta_kernel(double *norms, int k, double crit) {
         pass = pass && __ballot(!(nr <= crit * nA * nx)) == 0;
         for (int q = 0; q < min(64, k - c0); ++q) {
             const double eq = bcast_lane(e, q);
-            if (!(eq <= eta)) eta = eq;  // keeps NaN
+            if (!(eq <= eta) && !isnan(eta)) eta = eq;  // NaN stays
         }
     }
     if (lane == 0) {
@@ -307,7 +307,7 @@ RefineOut gmres_refine(hipStream_t s, const LowFactor &f, int64_t k, const doubl
         outer = std::max(outer, gmres_group(s, f, kc, B + c0, ldb, X + c0, ldx, g, sN.as<double>(), crit, &e, &conv,
                                             &inner));
         all = all && conv;
-        if (!(e <= eta)) eta = e;
+        if (!(e <= eta) && !std::isnan(eta)) eta = e;  // NaN stays
     }
     out.iterations = inner;
     out.eta = eta;
