@@ -1383,21 +1383,59 @@ int table_tile(int bytes, int64_t m, int64_t n, int64_t k) {
     return TILE_DEFAULT;
 }
 
-// gemm_direct_kernel where it beats the tiles through LDS: FP64, except
-// A B^T with aligned rows (51.7 TF through LDS, 49.9 TF direct at 4096^3: both
-// operands cost 16 lines a load; FP32, whose MFMA takes half the time for half
-// the bytes, lost everywhere), and enough tiles for the CUs (144 tiles, 1100 x
-// 1000 x 900: 69 against 87 us; 128 tiles, 1024^3: 75 against 67 us).  Returns
-// whether it took the product.
-constexpr int64_t DIRECT_FILL = 140;
+// The tile of a plain product's kernels through LDS: the tuned table's where it
+// has one, else large outputs take large tiles and smaller ones 64 x 64, so
+// that the launch still spreads over the 256 CUs.  FP64 that gemm_nn_kernel
+// takes has 128 x 64 (224 registers a wave against 392 at 128 x 128, so two
+// waves share a SIMD): 46 -> 53 TF at 8192^3.  A product beside the LU panels
+// keeps its measured 128 x 128 (the table is timed on an idle device; FP64 LU
+// at n = 8192 with 128 x 64: 75.2 against 72.4 ms, the panels slowed more than
+// the GEMM gained).
+int plain_tile(int bytes, bool nn, bool sharing, int64_t m, int64_t n, int64_t k) {
+    const int tile = sharing ? TILE_DEFAULT : table_tile(bytes, m, n, k);
+    if (tile != TILE_DEFAULT) return tile;
+    if (cdiv(m, 128) * cdiv(n, 128) < 512) return TILE_64x64;
+    return bytes == 8 && nn && !sharing ? TILE_128x64 : TILE_128x128;
+}
+
+// gemm_direct_kernel or the tiles through LDS, for an FP64 product on an idle
+// device: whichever the two's times say (us), one tile a CU a round.  Both are
+// bound by the matrix cores within a round, so what decides is how the output
+// divides: a direct tile has 64 x 128, of which n <= 64 wastes half, and 129
+// columns or a grid just past a round of the CUs a third, where 64 x 64 tiles
+// waste little.
+//   The times are fitted to 1043 products (m, n from 1 to 100000, k from 64 to
+// 4096, every transpose, rows aligned and not), where they choose the slower
+// kernel by more than 3% in 8 of the cases that the tiles win (6% at most);
+// taking the direct kernel from 140 tiles on had 361 slower ones, up to 1.8
+// times (32668 x 4 x 78: 9.7 against 17.4 us, 40000 x 64 x 256 36 against 57,
+// 9000 x 192 x 1024 92 against 134), and 7% more time over all.
+//   Aligned A B^T is not in it: 51.7 TF through LDS, 49.9 TF direct at 4096^3
+// (both operands cost 16 lines a load).  Nor is FP32, whose MFMA takes half the
+// time for half the bytes: it lost everywhere.
 constexpr int DIRECT_MIN_K = 64;
-bool gemm_direct(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k, double alpha, const double *A,
-                 int64_t lda, const double *B, int64_t ldb, double beta, double *C, int64_t ldc) {
+bool direct_is_faster(bool ta, bool tb, bool nn, int tile, int64_t m, int64_t n, int64_t k) {
+    auto rounds = [&](int64_t bm, int64_t bn) { return (double)cdiv(cdiv(m, bm) * cdiv(n, bn), 256); };
+    const double kk = (double)k;
+    // one transpose of the two: the operands cost fewer lines
+    const double direct = 3.2 + rounds(64, 128) * (3.9 + (ta != tb ? 0.0600 : 0.0645) * kk);
+    double tiles;
+    if (tile == TILE_64x64) {
+        // the first tiles of a CU hide each other's latency
+        const double r = rounds(64, 64), first[3] = {nn ? 0.059 : 0.066, nn ? 0.088 : 0.097, nn ? 0.119 : 0.131};
+        tiles = 1.5 + 2.0 * r + kk * (r <= 3 ? first[(int)r - 1] : r * (nn ? 0.0405 : 0.045));
+    } else if (tile == TILE_128x64) {
+        tiles = 1.5 + rounds(128, 64) * (3.0 + (nn ? 0.082 : 0.1) * kk);
+    } else {
+        tiles = 1.5 + rounds(128, 128) * (6.0 + 0.188 * kk);
+    }
+    return direct < tiles;
+}
+
+void launch_direct(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k, double alpha, const double *A,
+                   int64_t lda, const double *B, int64_t ldb, double beta, double *C, int64_t ldc) {
     constexpr int MT = 2, NT = 4;
-    const BatchStrides nob{1, 0, 0, 0, 0, 0, 0};
-    if (tb && nn_ok<double>(ta, tb, n, k, A, lda, B, ldb, nob)) return false;
     const int tiles_m = (int)cdiv(m, 32 * MT), tiles_n = (int)cdiv(n, 32 * NT);
-    if (k < DIRECT_MIN_K || (int64_t)tiles_m * tiles_n < DIRECT_FILL) return false;
     auto al = [](const void *p, int64_t ld) { return ((uintptr_t)p & 15) == 0 && ld % 2 == 0; };
     const bool vec = (ta || al(A, lda)) && (!tb || al(B, ldb));
     TimedRegion tr("gemm", s, 2.0 * (double)m * (double)n * (double)k);
@@ -1418,7 +1456,6 @@ bool gemm_direct(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t 
         LMX_DIRECT(true, true, false);
 #undef LMX_DIRECT
     LMX_LAUNCH_CHECK();
-    return true;
 }
 
 template <class T>
@@ -1429,56 +1466,30 @@ void gemm_impl(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k,
     if (m == 0 || n == 0) return;
     if (m > INT32_MAX / 2 || n > INT32_MAX / 2 || k > INT32_MAX / 2) fail_arg("gemm: dimension too large");
     const double flops = 2.0 * (double)m * (double)n * (double)k;
-    // A GEMM sharing its CUs with the LU panels keeps its measured tile (the
-    // table is timed on an idle device); the others take the tuned table's
-    // tile where it has one.
+    const BatchStrides nob{1, 0, 0, 0, 0, 0, 0};
+    const bool nn = nn_ok<T>(ta, tb, n, k, A, lda, B, ldb, nob);
+    const int tile = plain_tile((int)sizeof(T), nn, sharing, m, n, k);
     if constexpr (sizeof(T) == 8) {
         // beside the LU panels only where the product is the longer of the two
         // (FP64 LU n = 16384 141 -> 128 ms; at n = 8192 36.0 against 36.2 ms)
-        if ((!sharing || m > 8192) && lds_footprint == 0 && t_tile_override == TILE_DEFAULT &&
-            gemm_direct(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc))
+        if (!(tb && nn) && k >= DIRECT_MIN_K && lds_footprint == 0 && t_tile_override == TILE_DEFAULT &&
+            (sharing ? m > 8192 : direct_is_faster(ta, tb, nn, tile, m, n, k))) {
+            launch_direct(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
             return;
+        }
     }
-    const int tile = sharing ? TILE_DEFAULT : table_tile((int)sizeof(T), m, n, k);
-    if (tile != TILE_DEFAULT) {
-        const BatchStrides nob{1, 0, 0, 0, 0, 0, 0};
-        const bool big = tile != TILE_64x64;
-        TimedRegion tr(sizeof(T) == 8 ? (big ? "gemm" : "gemm64") : (big ? "sgemm" : "sgemm64"), s, flops);
-        if (tile == TILE_64x64)
-            launch_tile<T, 64, 64, 16>(s, ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C, ldc, 0, 1,
-                                       nob, lds_footprint);
-        else if (tile == TILE_128x64)
-            launch_tile<T, 128, 64, 16>(s, ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C, ldc, 0, 1,
-                                        nob, lds_footprint);
-        else
-            launch_tile<T, 128, 128, 16>(s, ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C, ldc, 0,
-                                         1, nob, lds_footprint);
-        return;
-    }
-    // The fixed rule: large outputs take 128 x 128 tiles, smaller ones
-    // 64 x 64 so the launch still spreads over the 256 CUs.  Each tile size
-    // is its own timing family.
-    int64_t big_tiles = cdiv(m, 128) * cdiv(n, 128);
-    if (big_tiles >= 512) {
-        TimedRegion tr(sizeof(T) == 8 ? "gemm" : "sgemm", s, flops);
-        const BatchStrides nob{1, 0, 0, 0, 0, 0, 0};
-        // FP64 NN below gemm_direct's limits, and aligned A B^T: 128 x 64
-        // tiles (224 registers a wave against 392 at 128 x 128, so two waves
-        // share a SIMD): 46 -> 53 TF at 8192^3.  A GEMM beside the LU panels
-        // keeps 128 x 128 where gemm_direct leaves it (m <= 8192): with
-        // 128 x 64 the panels slowed more than the GEMM gained (FP64 LU at
-        // n=8192: 75.2 against 72.4 ms).
-        if (sizeof(T) == 8 && !sharing && nn_ok<T>(ta, tb, n, k, A, lda, B, ldb, nob))
-            launch_tile<T, 128, 64, 16>(s, ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C, ldc, 0, 1,
-                                        nob, lds_footprint);
-        else
-            launch_tile<T, 128, 128, 16>(s, ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta,
-                                         C, ldc, 0, 1, nob, lds_footprint);
-    } else {
-        TimedRegion tr(sizeof(T) == 8 ? "gemm64" : "sgemm64", s, flops);
-        launch_tile<T, 64, 64, 16>(s, ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta,
-                                   C, ldc, 0, 1, BatchStrides{1, 0, 0, 0, 0, 0, 0}, lds_footprint);
-    }
+    // each tile size is its own timing family
+    const bool big = tile != TILE_64x64;
+    TimedRegion tr(sizeof(T) == 8 ? (big ? "gemm" : "gemm64") : (big ? "sgemm" : "sgemm64"), s, flops);
+    if (tile == TILE_64x64)
+        launch_tile<T, 64, 64, 16>(s, ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C, ldc, 0, 1, nob,
+                                   lds_footprint);
+    else if (tile == TILE_128x64)
+        launch_tile<T, 128, 64, 16>(s, ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C, ldc, 0, 1, nob,
+                                    lds_footprint);
+    else
+        launch_tile<T, 128, 128, 16>(s, ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C, ldc, 0, 1,
+                                     nob, lds_footprint);
 }
 
 template <class T>

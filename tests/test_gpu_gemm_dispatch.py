@@ -1,0 +1,41 @@
+"""Which kernel a product takes, by the timing family it is counted in, and
+its exact result (integer operands) on both sides of the rule."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def family(lmx, call):
+    """The families among `gemm` (large tiles) and `gemm64` that call() used."""
+    lmx.kernel_timing(True)
+    try:
+        lmx.kernel_timing_reset()
+        call()
+        return [f for f in ("gemm", "gemm64") if lmx.kernel_timing_get(f)[0] > 0]
+    finally:
+        lmx.kernel_timing(False)
+
+
+# 64 x 64 tiles where 64 x 128 would multiply padding or fill a round of the
+# 256 CUs badly: few columns, 129 - 192 columns, a grid just past a round, a
+# small k; the wave-by-wave kernel where its tiles divide the output well
+@pytest.mark.parametrize("m,n,k,tb,pad,want", [
+    (16384, 1, 64, "N", 0, "gemm64"), (9001, 16, 300, "N", 1, "gemm64"), (30000, 64, 128, "N", 0, "gemm64"),
+    (9000, 192, 256, "N", 0, "gemm64"), (17000, 50, 100, "T", 1, "gemm64"), (6000, 320, 500, "N", 0, "gemm64"),
+    (1500, 1500, 64, "N", 0, "gemm64"),
+    (2000, 1000, 777, "N", 0, "gemm"), (4096, 1024, 512, "N", 1, "gemm"), (8192, 256, 256, "N", 0, "gemm")])
+@pytest.mark.parametrize("ta", ["N", "T"])
+def test_fp64_tiles(lmx_gpu, m, n, k, tb, pad, want, ta):
+    import torch
+
+    def operand(rows, cols, seed):
+        v = torch.tensor(np.random.default_rng(seed).integers(-8, 9, (rows, cols)).astype(float), device="cuda")
+        return torch.nn.functional.pad(v, (0, pad))[:, :cols]
+
+    A = operand(*((k, m) if ta == "T" else (m, k)), 1)
+    B = operand(*((n, k) if tb == "T" else (k, n)), 2)
+    C = torch.empty(m, n, dtype=torch.float64, device="cuda")
+    assert family(lmx_gpu, lambda: lmx_gpu.dgemm_dev(A, B, C, transa=ta, transb=tb)) == [want]
+    a, b = A.cpu().numpy(), B.cpu().numpy()
+    np.testing.assert_array_equal(C.cpu().numpy(), (a.T if ta == "T" else a) @ (b.T if tb == "T" else b))
