@@ -1421,9 +1421,13 @@ bool direct_is_faster(bool ta, bool tb, bool nn, int tile, int64_t m, int64_t n,
     const double direct = 3.2 + rounds(64, 128) * (3.9 + (ta != tb ? 0.0600 : 0.0645) * kk);
     double tiles;
     if (tile == TILE_64x64) {
+        // a round or less is gemm_ksplit_kernel's (16 x 16 x 8192: 30 us, one
+        // direct tile 490)
+        const double r = rounds(64, 64);
+        if (r < 2) return false;
         // the first tiles of a CU hide each other's latency
-        const double r = rounds(64, 64), first[3] = {nn ? 0.059 : 0.066, nn ? 0.088 : 0.097, nn ? 0.119 : 0.131};
-        tiles = 1.5 + 2.0 * r + kk * (r <= 3 ? first[(int)r - 1] : r * (nn ? 0.0405 : 0.045));
+        const double first[2] = {nn ? 0.088 : 0.097, nn ? 0.119 : 0.131};
+        tiles = 1.5 + 2.0 * r + kk * (r <= 3 ? first[(int)r - 2] : r * (nn ? 0.0405 : 0.045));
     } else if (tile == TILE_128x64) {
         tiles = 1.5 + rounds(128, 64) * (3.0 + (nn ? 0.082 : 0.1) * kk);
     } else {

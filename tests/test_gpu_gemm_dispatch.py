@@ -24,6 +24,8 @@ def family(lmx, call):
     (16384, 1, 64, "N", 0, "gemm64"), (9001, 16, 300, "N", 1, "gemm64"), (30000, 64, 128, "N", 0, "gemm64"),
     (9000, 192, 256, "N", 0, "gemm64"), (17000, 50, 100, "T", 1, "gemm64"), (6000, 320, 500, "N", 0, "gemm64"),
     (1500, 1500, 64, "N", 0, "gemm64"),
+    # a round of 64 x 64 tiles or less: the split-k kernel
+    (16, 16, 8192, "N", 0, "gemm64"), (33, 300, 8000, "T", 1, "gemm64"), (500, 500, 2000, "N", 1, "gemm64"),
     (2000, 1000, 777, "N", 0, "gemm"), (4096, 1024, 512, "N", 1, "gemm"), (8192, 256, 256, "N", 0, "gemm")])
 @pytest.mark.parametrize("ta", ["N", "T"])
 def test_fp64_tiles(lmx_gpu, m, n, k, tb, pad, want, ta):
