@@ -483,7 +483,7 @@ void potrf_lookahead(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_inf
         T *A21 = A11 + kb * lda;
         T *X = (k0 / nb) % 2 ? sy.as<T>() : sx.as<T>();
         diag_block<T>(s, bf16, kb, A11, lda, k0, d_info, WT, tmp);
-        if (rest > 0) gemm(s, false, false, rest, kb, kb, T(1), A21, lda, WT, BLK, T(0), X, kb);
+        if (rest > 0) gemm_chain<T>(s, rest, kb, kb, T(1), A21, lda, WT, BLK, T(0), X, kb);
         // The trailing SYRK may start once the panel is in place: it and
         // the next block column's update below touch different elements.
         // Recording `ready` here keeps the event markers out of the gap

@@ -19,6 +19,7 @@
 // lane l sit in column l%16 at rows 4*(l/16) + r for f32 but at rows
 // l/16 + 4*r for f64 (measured on gfx950); acc_row() encodes both.
 #include "common.hpp"
+#include "gemm_rules.hpp"
 #include "kernels.hpp"
 
 namespace lmx {
@@ -1257,8 +1258,6 @@ bool nn_ok(bool ta, bool tb, int64_t n, int64_t k, const T *A, int64_t lda, cons
            bs.a1 % E == 0 && bs.a2 % E == 0 && bs.b1 % E == 0 && bs.b2 % E == 0;
 }
 
-// Tile shapes of the plain (non-batched, non-SYRK) GEMM dispatch.
-enum GemmTile { TILE_DEFAULT = 0, TILE_64x64 = 1, TILE_128x64 = 2, TILE_128x128 = 3 };
 thread_local int t_tile_override = TILE_DEFAULT;
 
 template <class T, int MT, int NT, bool VEC>
@@ -1281,27 +1280,23 @@ void launch_ksplit(hipStream_t s, bool ta, bool tb, int m, int n, int k, T alpha
     LMX_LAUNCH_CHECK();
 }
 
-// gemm_ksplit_kernel with the largest tile that still gives KS_FILL
-// workgroups (one a CU), else the smallest.
-constexpr int64_t KS_FILL = 256;
-constexpr int KS_MIN_K = 48;
 template <class T>
-void gemm_ksplit(hipStream_t s, bool ta, bool tb, int m, int n, int k, T alpha, const T *A, int64_t lda, const T *B,
-                 int64_t ldb, T beta, T *C, int64_t ldc, int lower, int batch, const BatchStrides &bs) {
+void gemm_ksplit(hipStream_t s, const KsTile &t, bool ta, bool tb, int m, int n, int k, T alpha, const T *A,
+                 int64_t lda, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, int lower, int batch,
+                 const BatchStrides &bs) {
     // 16-byte loads along k: every row of an operand whose k runs along
     // memory starts on a 16-byte boundary (its chunks then do too)
     constexpr int E = V16<T>::N;
     auto al = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
     const bool vec = (ta || (al(A) && lda % E == 0 && bs.a1 % E == 0 && bs.a2 % E == 0)) &&
                      (!tb || (al(B) && ldb % E == 0 && bs.b1 % E == 0 && bs.b2 % E == 0));
-    const int64_t t16 = cdiv(m, 16), t32 = cdiv(m, 32), u32 = cdiv(n, 32);
 #define LMX_KSPLIT(MT_, NT_)                                                                                    \
     (vec ? launch_ksplit<T, MT_, NT_, true>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower, batch, bs) \
          : launch_ksplit<T, MT_, NT_, false>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower, batch,    \
                                              bs))
-    if ((lower ? t32 * u32 / 2 : t32 * u32) * batch >= KS_FILL)
+    if (t.mt == 2)
         LMX_KSPLIT(2, 2);
-    else if (!lower && t16 * u32 * batch >= KS_FILL)
+    else if (t.nt == 2)
         LMX_KSPLIT(1, 2);
     else
         LMX_KSPLIT(1, 1);
@@ -1312,16 +1307,23 @@ template <class T, int BM, int BN, int BK>
 void launch_tile(hipStream_t s, bool ta, bool tb, int m, int n, int k, T alpha, const T *A,
                  int64_t lda, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, int lower = 0,
                  int batch = 1, BatchStrides bs = BatchStrides{1, 0, 0, 0, 0, 0, 0}, size_t lds_footprint = 0,
-                 bool nn_sharing = false) {
+                 bool nn_sharing = false, bool chain = false) {
     int tiles_m = (int)cdiv(m, BM), tiles_n = (int)cdiv(n, BN);
     dim3 grid(lower ? lower_tiles(tiles_m, tiles_n) : tiles_m * tiles_n, (unsigned)batch), block(256);
-    // Fewer 64 x 64 tiles than CUs: the split-k kernel (KS_MIN_K: with two
-    // 16-k chunks most of its waves would have nothing to do).
+    const bool nn = nn_ok<T>(ta, tb, n, k, A, lda, B, ldb, bs);
+    // Fewer 64 x 64 tiles than CUs: the split-k kernel where it is faster
+    // (KS_MIN_K: with two 16-k chunks most of its waves would have nothing to
+    // do).  On a factorisation's chain, beside another stream's update, always:
+    // its many waves get more of the CUs that the two share (FP64 Cholesky
+    // n = 8192: 9.30 against 9.70 ms with the rule for an idle device).
     if constexpr (BM == 64 && BN == 64) {
         if (lds_footprint == 0 && t_tile_override == TILE_DEFAULT && k >= KS_MIN_K &&
             (int64_t)grid.x * batch < KS_FILL) {
-            gemm_ksplit<T>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower, batch, bs);
-            return;
+            const KsTile t = ksplit_tile(m, n, lower != 0, batch);
+            if (chain || ksplit_is_faster((int)sizeof(T), t, nn, tb, k)) {
+                gemm_ksplit<T>(s, t, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower, batch, bs);
+                return;
+            }
         }
     }
     // lds_footprint: the LDS one workgroup should hold in all (its tiles plus
@@ -1330,7 +1332,7 @@ void launch_tile(hipStream_t s, bool ta, bool tb, int m, int n, int k, T alpha, 
     // kernel: the NN kernel is faster on its own but slows those panels more
     // (FP32 LU at n=16384: 155 against 151 ms).
     const bool sharing = lds_footprint > 0 && sizeof(T) == 4 && !nn_sharing;
-    if (!sharing && nn_ok<T>(ta, tb, n, k, A, lda, B, ldb, bs)) {
+    if (!sharing && nn) {
         const size_t st = gemm_nn_lds<T, BM, BN>(), reserve = lds_footprint > st ? lds_footprint - st : 0;
         if (tb)
             hipLaunchKernelGGL((gemm_nn_kernel<T, BM, BN, true>), grid, block, reserve, s, m, n, k, alpha, A, lda, B,
@@ -1398,44 +1400,6 @@ int plain_tile(int bytes, bool nn, bool sharing, int64_t m, int64_t n, int64_t k
     return bytes == 8 && nn && !sharing ? TILE_128x64 : TILE_128x128;
 }
 
-// gemm_direct_kernel or the tiles through LDS, for an FP64 product on an idle
-// device: whichever the two's times say (us), one tile a CU a round.  Both are
-// bound by the matrix cores within a round, so what decides is how the output
-// divides: a direct tile has 64 x 128, of which n <= 64 wastes half, and 129
-// columns or a grid just past a round of the CUs a third, where 64 x 64 tiles
-// waste little.
-//   The times are fitted to 1043 products (m, n from 1 to 100000, k from 64 to
-// 4096, every transpose, rows aligned and not), where they choose the slower
-// kernel by more than 3% in 8 of the cases that the tiles win (6% at most);
-// taking the direct kernel from 140 tiles on had 361 slower ones, up to 1.8
-// times (32668 x 4 x 78: 9.7 against 17.4 us, 40000 x 64 x 256 36 against 57,
-// 9000 x 192 x 1024 92 against 134), and 7% more time over all.
-//   Aligned A B^T is not in it: 51.7 TF through LDS, 49.9 TF direct at 4096^3
-// (both operands cost 16 lines a load).  Nor is FP32, whose MFMA takes half the
-// time for half the bytes: it lost everywhere.
-constexpr int DIRECT_MIN_K = 64;
-bool direct_is_faster(bool ta, bool tb, bool nn, int tile, int64_t m, int64_t n, int64_t k) {
-    auto rounds = [&](int64_t bm, int64_t bn) { return (double)cdiv(cdiv(m, bm) * cdiv(n, bn), 256); };
-    const double kk = (double)k;
-    // one transpose of the two: the operands cost fewer lines
-    const double direct = 3.2 + rounds(64, 128) * (3.9 + (ta != tb ? 0.0600 : 0.0645) * kk);
-    double tiles;
-    if (tile == TILE_64x64) {
-        // a round or less is gemm_ksplit_kernel's (16 x 16 x 8192: 30 us, one
-        // direct tile 490)
-        const double r = rounds(64, 64);
-        if (r < 2) return false;
-        // the first tiles of a CU hide each other's latency
-        const double first[2] = {nn ? 0.088 : 0.097, nn ? 0.119 : 0.131};
-        tiles = 1.5 + 2.0 * r + kk * (r <= 3 ? first[(int)r - 2] : r * (nn ? 0.0405 : 0.045));
-    } else if (tile == TILE_128x64) {
-        tiles = 1.5 + rounds(128, 64) * (3.0 + (nn ? 0.082 : 0.1) * kk);
-    } else {
-        tiles = 1.5 + rounds(128, 128) * (6.0 + 0.188 * kk);
-    }
-    return direct < tiles;
-}
-
 void launch_direct(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k, double alpha, const double *A,
                    int64_t lda, const double *B, int64_t ldb, double beta, double *C, int64_t ldc) {
     constexpr int MT = 2, NT = 4;
@@ -1465,7 +1429,7 @@ void launch_direct(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_
 template <class T>
 void gemm_impl(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k, T alpha,
                const T *A, int64_t lda, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, size_t lds_footprint = 0,
-               bool sharing = false) {
+               bool sharing = false, bool chain = false) {
     if (m < 0 || n < 0 || k < 0) fail_arg("gemm: negative dimension");
     if (m == 0 || n == 0) return;
     if (m > INT32_MAX / 2 || n > INT32_MAX / 2 || k > INT32_MAX / 2) fail_arg("gemm: dimension too large");
@@ -1487,7 +1451,7 @@ void gemm_impl(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k,
     TimedRegion tr(sizeof(T) == 8 ? (big ? "gemm" : "gemm64") : (big ? "sgemm" : "sgemm64"), s, flops);
     if (tile == TILE_64x64)
         launch_tile<T, 64, 64, 16>(s, ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C, ldc, 0, 1, nob,
-                                   lds_footprint);
+                                   lds_footprint, false, chain);
     else if (tile == TILE_128x64)
         launch_tile<T, 128, 64, 16>(s, ta, tb, (int)m, (int)n, (int)k, alpha, A, lda, B, ldb, beta, C, ldc, 0, 1, nob,
                                     lds_footprint);
@@ -1579,7 +1543,8 @@ void syrk_trap(hipStream_t s, int64_t m, int64_t n, int64_t k, T alpha, const T 
     if (m > INT32_MAX / 2 || k > INT32_MAX / 2) fail_arg("syrk_trap: dimension too large");
     const double elems = (double)n * (double)(n + 1) / 2 + (double)(m - n) * (double)n;
     TimedRegion tr(sizeof(T) == 8 ? "gemm64" : "sgemm64", s, 2.0 * elems * (double)k);
-    launch_tile<T, 64, 64, 16>(s, false, true, (int)m, (int)n, (int)k, alpha, A, lda, A, lda, beta, C, ldc, 1);
+    launch_tile<T, 64, 64, 16>(s, false, true, (int)m, (int)n, (int)k, alpha, A, lda, A, lda, beta, C, ldc, 1, 1,
+                               BatchStrides{1, 0, 0, 0, 0, 0, 0}, 0, false, true);
 }
 template void syrk_trap<double>(hipStream_t, int64_t, int64_t, int64_t, double, const double *, int64_t, double,
                                 double *, int64_t);
@@ -1597,6 +1562,16 @@ void gemm(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64_t k, floa
           int64_t ldc) {
     gemm_impl<float>(s, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
 }
+
+template <class T>
+void gemm_chain(hipStream_t s, int64_t m, int64_t n, int64_t k, T alpha, const T *A, int64_t lda, const T *B,
+                int64_t ldb, T beta, T *C, int64_t ldc) {
+    gemm_impl<T>(s, false, false, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, 0, false, true);
+}
+template void gemm_chain<double>(hipStream_t, int64_t, int64_t, int64_t, double, const double *, int64_t,
+                                 const double *, int64_t, double, double *, int64_t);
+template void gemm_chain<float>(hipStream_t, int64_t, int64_t, int64_t, float, const float *, int64_t, const float *,
+                                int64_t, float, float *, int64_t);
 
 template <class T>
 void gemm_sharing(hipStream_t s, int64_t m, int64_t n, int64_t k, T alpha, const T *A, int64_t lda, const T *B,

@@ -43,6 +43,12 @@ template <class T>
 void gemm_sharing(hipStream_t s, int64_t m, int64_t n, int64_t k, T alpha, const T *A, int64_t lda, const T *B,
                   int64_t ldb, T beta, T *C, int64_t ldc, size_t lds_footprint);
 
+// C = alpha A B + beta C on a factorisation's chain, beside an update on
+// another stream.
+template <class T>
+void gemm_chain(hipStream_t s, int64_t m, int64_t n, int64_t k, T alpha, const T *A, int64_t lda, const T *B,
+                int64_t ldb, T beta, T *C, int64_t ldc);
+
 // Batched C_z = alpha A_z B_z + beta C_z (no transposes) for z = zk nb1 + zp,
 // zk < nb2, zp < nb1; entry z's matrices start at zk x2 + zp x1 elements
 // from A, B, C.
