@@ -1037,7 +1037,6 @@ bool bf16_vec_ok(bool ta, bool tb, int64_t m, int64_t n, int64_t k, const S *A, 
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
 constexpr int BX_K = 64, BX_SK = 72;
-constexpr int64_t BX_MIN_TILES = 100;
 
 template <bool KC, int NT>
 struct BxTile {
@@ -1166,19 +1165,12 @@ __global__ __launch_bounds__(2 * BT) void gemm_bf16_large_kernel(int m, int n, i
         }
 }
 
-// The tile gemm_bf16_large_kernel takes a product with, 0 where it does not:
-// every 16-byte vector has to be wholly inside or outside its operand and
-// aligned.
-int bf16_large_tile(bool ta, bool tb, int64_t m, int64_t n, int64_t k, const unsigned short *A, int64_t lda,
-                    const unsigned short *B, int64_t ldb) {
+// Whether gemm_bf16_large_kernel can take a product: every 16-byte vector has
+// to be wholly inside or outside its operand and aligned.
+bool bf16_large_ok(bool ta, bool tb, int64_t m, int64_t n, int64_t k, const unsigned short *A, int64_t lda,
+                   const unsigned short *B, int64_t ldb) {
     auto al = [](const void *p) { return ((uintptr_t)p & 15) == 0; };
-    if (!(al(A) && al(B) && lda % 8 == 0 && ldb % 8 == 0 && (ta ? m : k) % 8 == 0 && (tb ? k : n) % 8 == 0)) return 0;
-    // rounds over the chip, one 256 x 256 tile a CU or two 128 x 128; a round
-    // of the former takes 40 / 23 of the latter's time (2048 x 4096 x 8192 NT:
-    // 206 against 160 us, one round each)
-    const int64_t t256 = cdiv(m, 256) * cdiv(n, 256), t128 = cdiv(m, 128) * cdiv(n, 128);
-    if (t128 < BX_MIN_TILES) return 0;  // the 64 x 64 tiles spread better (1024^3 NT: 15.0 against 19.3 us)
-    return 40 * cdiv(t256, 256) <= 23 * cdiv(t128, 512) ? 256 : 128;
+    return al(A) && al(B) && lda % 8 == 0 && ldb % 8 == 0 && (ta ? m : k) % 8 == 0 && (tb ? k : n) % 8 == 0;
 }
 
 template <int BT>
@@ -1214,7 +1206,8 @@ void gemm_bf16_impl(hipStream_t s, bool ta, bool tb, int64_t m, int64_t n, int64
     const int64_t big = lower ? cdiv(m, 128) * (cdiv(m, 128) + 1) / 2 : cdiv(m, 128) * cdiv(n, 128);
     const int M = (int)m, N = (int)n, K = (int)k;
     if constexpr (sizeof(S) == 2) {
-        const int tile = lower ? 0 : bf16_large_tile(ta, tb, m, n, k, A, lda, B, ldb);
+        const int tile =
+            !lower && bf16_large_ok(ta, tb, m, n, k, A, lda, B, ldb) ? bf16_large_tile(ta, tb, m, n, k) : 0;
         if (tile == 256) return launch_bf16_large<256>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
         if (tile == 128) return launch_bf16_large<128>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
     }

@@ -95,4 +95,50 @@ inline bool direct_is_faster(bool ta, bool tb, bool nn, int tile, int64_t m, int
     return direct < tiles;
 }
 
+// The tile (256 or 128) that gemm_bf16_large_kernel takes a product with, 0
+// where the 128 x 128 x 32 and 64 x 64 x 32 tiles of gemm_bf16_kernel are the
+// faster ones: whichever the times say (us, `w` million elements of C).
+//   Rounds over the chip: one 256 x 256 tile a CU or two 128 x 128; a round of
+// the former takes 40 / 23 of the latter's time (2048 x 4096 x 8192 NT: 206
+// against 160 us, one round each).  Below BX_MIN_TILES the 64 x 64 tiles spread
+// better (1024^3 NT: 15.0 against 19.3 us).  A large tile's start and its C
+// cost 5 to 12 us a round, which its k steps have to pay for: 2048 x 2048 x 8
+// took 8.4 us in place of 6.5, 13216 x 40 x 8 6.9 in place of 3.8.
+//   The times are fitted to 637 products (m, n from 8 to 65536, k from 8 to
+// 8192, every transpose), where they choose the slower kernel by more than 3%
+// in 10 of the cases that the smaller steps win (14% at most); the large tiles
+// for all of them were slower in 328, up to 1.83 times, and gained nothing over
+// all, against 11% now.
+constexpr int64_t BX_MIN_TILES = 100;
+inline int bf16_large_tile(bool ta, bool tb, int64_t m, int64_t n, int64_t k) {
+    const int64_t t256 = rule_cdiv(m, 256) * rule_cdiv(n, 256), t128 = rule_cdiv(m, 128) * rule_cdiv(n, 128);
+    if (t128 < BX_MIN_TILES) return 0;
+    const int tile = 40 * rule_cdiv(t256, 256) <= 23 * rule_cdiv(t128, 512) ? 256 : 128;
+    // us of one round per k: NN, NT, TN, TT
+    static const double first256[4] = {0.0307, 0.0291, 0.0342, 0.0312}, more256[4] = {0.0343, 0.0330, 0.0355, 0.0345},
+                        one128[4] = {0.0147, 0.0129, 0.0177, 0.0151}, two128[4] = {0.0184, 0.0166, 0.0214, 0.0194},
+                        small128[4] = {0.0145, 0.0122, 0.0190, 0.0150},
+                        small64[3][4] = {{0.0170, 0.0136, 0.0207, 0.0172},
+                                         {0.0084, 0.0078, 0.0105, 0.0091},
+                                         {0.0074, 0.0053, 0.0097, 0.0074}};
+    const int f = 2 * ta + tb;
+    const double kk = (double)k, w = (double)m * (double)n * 1e-6;
+    double large, small;
+    if (tile == 256) {
+        const double r = (double)rule_cdiv(t256, 256);
+        large = r == 1 ? 12.2 + 0.11 * w + first256[f] * kk : 0.9 * w + r * more256[f] * kk;
+    } else if (t128 <= 256) {  // one tile a CU
+        large = 4.5 + 1.05 * w + one128[f] * kk;
+    } else {
+        large = 5.0 + 0.77 * w + (double)rule_cdiv(t128, 512) * two128[f] * kk;
+    }
+    if (t128 >= 512) {
+        small = 4.3 + 0.68 * w + (double)rule_cdiv(t128, 256) * small128[f] * kk;
+    } else {
+        const int64_t r = rule_cdiv(rule_cdiv(m, 64) * rule_cdiv(n, 64), 256);
+        small = 2.7 + (r < 5 ? 0.9 : 0.68) * w + (double)r * small64[r < 3 ? r - 1 : 2][f] * kk;
+    }
+    return large < small ? tile : 0;
+}
+
 }  // namespace lmx

@@ -17,7 +17,8 @@ int main() {
     int bytes, ta, tb, nn, tile;
     long m, n, k;
     while (scanf("%15s %d %d %d %d %d %ld %ld %ld", rule, &bytes, &ta, &tb, &nn, &tile, &m, &n, &k) == 9)
-        printf("%d\n", !strcmp(rule, "split") ? (int)ksplit_is_faster(bytes, ksplit_tile(m, n, false, 1), nn, tb, k)
+        printf("%d\n", !strcmp(rule, "bf16")    ? bf16_large_tile(ta, tb, m, n, k) > 0
+                       : !strcmp(rule, "split") ? (int)ksplit_is_faster(bytes, ksplit_tile(m, n, false, 1), nn, tb, k)
                                               : (int)direct_is_faster(ta, tb, nn, tile, m, n, k));
 }
 """
@@ -47,6 +48,15 @@ DIRECT = [
     ("d", "NN", 0, 7144, 144, 1664, 144.3, 110.8), ("d", "TN", 0, 668, 1898, 1576, 158.8, 101.5),
     ("d", "NT", 1, 1025, 1100, 300, 34.1, 25.7), ("d", "TN", 0, 1999, 1001, 777, 90.0, 68.8),
 ]
+# BF16, aligned: the same, us with 32 k a step, us on the large tiles
+BF16 = [("b", f, 0, *rest) for f, *rest in [
+    ("NT", 2048, 2048, 64, 7.0, 8.4), ("NT", 38520, 24, 208, 6.9, 8.6), ("NT", 1048, 29528, 16, 26.7, 32.2),
+    ("TN", 408, 22216, 16, 11.5, 13.8), ("NT", 392, 7440, 32, 5.8, 7.7), ("NT", 3344, 416, 136, 5.8, 8.5),
+    ("NN", 896, 3512, 24, 5.9, 7.9), ("NT", 8, 34184, 256, 6.6, 8.2), ("TN", 24640, 1976, 24, 38.3, 48.8),
+    ("TT", 13216, 40, 8, 3.8, 6.9), ("NN", 2048, 2048, 8, 6.6, 8.4), ("NT", 16384, 64, 256, 6.3, 8.9),
+    ("NT", 4096, 4096, 256, 28.3, 20.1), ("TN", 24704, 184, 1224, 64.7, 35.1), ("NT", 136, 30760, 7576, 371.1, 178.9),
+    ("TT", 10376, 6696, 1104, 312.6, 243.5), ("NT", 14824, 904, 560, 44.7, 30.6), ("NN", 64, 65536, 256, 17.9, 14.3),
+    ("TT", 7280, 1496, 1576, 88.5, 65.5), ("TN", 152, 20272, 552, 25.5, 19.5), ("NN", 8192, 8192, 8192, 2390, 1090)]]
 
 
 def aligned(t, f, pad, m, n, k):
@@ -69,7 +79,7 @@ def choose(tmp_path_factory):
     return run
 
 
-@pytest.mark.parametrize("rule,cases", [("split", SPLIT), ("direct", DIRECT)])
+@pytest.mark.parametrize("rule,cases", [("split", SPLIT), ("direct", DIRECT), ("bf16", BF16)])
 def test_the_faster_kernel_is_chosen(choose, rule, cases):
     lines = []
     for t, f, pad, m, n, k, _, _ in cases:

@@ -41,3 +41,24 @@ def test_fp64_tiles(lmx_gpu, m, n, k, tb, pad, want, ta):
     assert family(lmx_gpu, lambda: lmx_gpu.dgemm_dev(A, B, C, transa=ta, transb=tb)) == [want]
     a, b = A.cpu().numpy(), B.cpu().numpy()
     np.testing.assert_array_equal(C.cpu().numpy(), (a.T if ta == "T" else a) @ (b.T if tb == "T" else b))
+
+
+# deep enough for the BF16 tiles of 128 (the first two) and 256, with remainders
+# in m, n and k
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
+@pytest.mark.parametrize("m,n,k,pad,beta", [(1288, 1304, 2056, 0, 0.0), (1160, 2440, 2120, 8, 3.0),
+                                            (3080, 3000, 1032, 0, 3.0), (2568, 4104, 904, 16, 0.0)])
+def test_bf16_large_tiles_exact(lmx_gpu, m, n, k, pad, beta, ta, tb):
+    import torch
+
+    def operand(rows, cols, seed, dtype):
+        v = torch.tensor(np.random.default_rng(seed).integers(-8, 9, (rows, cols)), device="cuda").to(dtype)
+        return torch.nn.functional.pad(v, (0, pad))[:, :cols]
+
+    A = operand(*((k, m) if ta == "T" else (m, k)), 1, torch.bfloat16)
+    B = operand(*((n, k) if tb == "T" else (k, n)), 2, torch.bfloat16)
+    C = operand(m, n, 3, torch.float32)
+    a, b, c = A.double().cpu().numpy(), B.double().cpu().numpy(), C.double().cpu().numpy()
+    lmx_gpu.gemm_bf16_dev(A, B, C, alpha=2.0, beta=beta, transa=ta, transb=tb)
+    want = 2 * ((a.T if ta == "T" else a) @ (b.T if tb == "T" else b)) + beta * c
+    np.testing.assert_array_equal(C.cpu().numpy().astype(float), want)
