@@ -194,10 +194,10 @@ struct TieRule {
     __device__ static int wave_pick(int v) { return TL ? wave_max_int(v) : wave_min(v); }
 };
 
-// The workgroup's best of the PW wave slots: largest value, the tie rule's
-// id on ties.  All slots are loaded before any comparison: compared as they
+// The workgroup's best of the PW wave slots (tournament): largest value, the
+// lowest id on ties.  All slots are loaded before any comparison: compared as they
 // are read, every step waits for its own LDS round trip.
-template <class T, bool TL = false>
+template <class T>
 __device__ __forceinline__ void wg_select(const T *vals, const int *ids, T &best, int &bid, int &bw) {
     T v[PW];
     int id[PW];
@@ -211,7 +211,7 @@ __device__ __forceinline__ void wg_select(const T *vals, const int *ids, T &best
     bw = 0;
 #pragma unroll
     for (int x = 1; x < PW; ++x) {
-        const bool take = v[x] > best || (v[x] == best && TieRule<TL>::better(id[x], bid));
+        const bool take = v[x] > best || (v[x] == best && TieRule<false>::better(id[x], bid));
         best = take ? v[x] : best;
         bid = take ? id[x] : bid;
         bw = take ? x : bw;
@@ -576,8 +576,8 @@ struct RowVec<double> {
 // (rows relative to the panel's first row): columns [c0, c1) and [c2, c3)
 // of G, and the permutation vector perm when not null; pairs_out receives
 // the move list (rows absolute) for the columns left for later.
-//   With u12 set, rows 0 .. KB - 1 of columns [c2, c3) (B12 of a full
-// panel) receive U12 = L11^{-1} B12 instead of the gathered B12.
+//   Rows 0 .. KB - 1 of columns [c2, c3) (B12, beside a panel of full width)
+// receive U12 = L11^{-1} B12 instead of the gathered B12.
 template <class T>
 struct PanelGather {
     T *G;
@@ -585,7 +585,6 @@ struct PanelGather {
     int c0, c1, c2, c3;
     int32_t *perm;
     int32_t *pairs_out;
-    int u12;
 };
 
 // The wave's 128 panel rows between memory and registers, 64 bytes of every
@@ -788,7 +787,6 @@ __attribute__((amdgpu_waves_per_eu(PanelShape<T>::MIN_WAVES_PER_SIMD))) void get
     }
     if (!rows) return;
     const int n1 = gx.c1 - gx.c0, ncols = n1 + (gx.c3 - gx.c2);
-    const bool u12 = gx.u12 != 0 && kb == KB;
     for (int c0 = (wave * P + w) * 64; c0 < ncols; c0 += S::WAVES * P * 64) {
         const int c = c0 + lane, cc = min(c, ncols - 1);
         T *col = gx.G + (cc < n1 ? gx.c0 + cc : gx.c2 + (cc - n1));
@@ -796,7 +794,7 @@ __attribute__((amdgpu_waves_per_eu(PanelShape<T>::MIN_WAVES_PER_SIMD))) void get
 #pragma unroll
         for (int e = 0; e < 2 * KB; ++e)
             x[e] = col[(int64_t)__builtin_amdgcn_readlane(src, e) * gx.ldg];  // past cnt: row 0, not used
-        if (u12 && cc >= n1) {
+        if (kb == KB && cc >= n1) {
 #pragma unroll
             for (int k = 0; k < KB - 1; ++k) {
 #pragma unroll
@@ -1613,7 +1611,7 @@ void getrf_impl(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_ipiv, in
                 }
             }
             if (!tslu_done) {
-                const PanelGather<T> gx{A + (int64_t)s0 * lda, lda, k0, s0, s0 + sb, k0 + nbw, perm_s, pairs_s, 1};
+                const PanelGather<T> gx{A + (int64_t)s0 * lda, lda, k0, s0, s0 + sb, k0 + nbw, perm_s, pairs_s};
                 launch_panel<T>(s, m, sb, P0, lda, s0, d_ipiv, d_info, sy, base, tie_last, gx);
             }
             const int rest = k0 + nbw - (s0 + sb);
