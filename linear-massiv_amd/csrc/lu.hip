@@ -1246,14 +1246,17 @@ __global__ __launch_bounds__(256) void row_gather_kernel(T *__restrict__ X, int6
 constexpr int PAIR_STRIDE = 4 * KB + 4;
 constexpr int PANELS_PER_BLOCK = NB_OUTER / KB;
 // LDS footprint of a workgroup of the lookahead's trailing GEMM: 64000
-// bytes keep the FP32 GEMM at two workgroups per CU, leaving a CU room for
-// an FP32 panel workgroup (21 KB) or inner-update workgroup (33 KB); the
-// FP64 GEMM tiles already hold that much, and a reserve would cost them
-// half their occupancy (0: none).
+// bytes keep the FP32 GEMM at two workgroups per CU, which leaves a CU room for
+// an FP32 panel workgroup (25.2 KB) or inner-update workgroup (8 KB).  The
+// tournament's kernels (512 x 33 numbers staged, 70 KB) do not fit beside two
+// and wait for GEMM tiles to end.  The FP64 GEMM tiles already hold that much,
+// and a reserve would cost them half their occupancy (0: none).
 template <class T>
 constexpr size_t aux_gemm_lds_footprint() {
     return sizeof(T) == 4 ? 64000 : 0;
 }
+static_assert(2 * aux_gemm_lds_footprint<float>() + sizeof(PanelLds<float>) <= 160 * 1024,
+              "an FP32 panel workgroup has to find room beside two of the GEMM's");
 // The BF16 lookahead GEMM's workgroup (80 KB of tiles) held to one per CU.
 constexpr size_t BF16_SHARING_LDS = 96 * 1024;
 template <class T>
