@@ -1306,14 +1306,15 @@ void launch_tile(hipStream_t s, bool ta, bool tb, int m, int n, int k, T alpha, 
     const bool nn = nn_ok<T>(ta, tb, n, k, A, lda, B, ldb, bs);
     // Fewer 64 x 64 tiles than CUs: the split-k kernel where it is faster
     // (KS_MIN_K: with two 16-k chunks most of its waves would have nothing to
-    // do).  On a factorisation's chain, beside another stream's update, always:
-    // its many waves get more of the CUs that the two share (FP64 Cholesky
-    // n = 8192: 9.30 against 9.70 ms with the rule for an idle device).
+    // do).  Always for a batch (the rule's times are of single products) and
+    // inside a factorisation, beside another stream's kernels, where its many
+    // waves get more of the CUs that the two share: FP64 Cholesky n = 8192 9.30
+    // against 9.70 ms with the rule for an idle device (LU 36.0 ms either way).
     if constexpr (BM == 64 && BN == 64) {
         if (lds_footprint == 0 && t_tile_override == TILE_DEFAULT && k >= KS_MIN_K &&
             (int64_t)grid.x * batch < KS_FILL) {
             const KsTile t = ksplit_tile(m, n, lower != 0, batch);
-            if (chain || ksplit_is_faster((int)sizeof(T), t, nn, tb, k)) {
+            if (chain || batch > 1 || ksplit_is_faster((int)sizeof(T), t, nn, tb, k)) {
                 gemm_ksplit<T>(s, t, ta, tb, m, n, k, alpha, A, lda, B, ldb, beta, C, ldc, lower, batch, bs);
                 return;
             }

@@ -43,8 +43,8 @@ template <class T>
 void gemm_sharing(hipStream_t s, int64_t m, int64_t n, int64_t k, T alpha, const T *A, int64_t lda, const T *B,
                   int64_t ldb, T beta, T *C, int64_t ldc, size_t lds_footprint);
 
-// C = alpha A B + beta C on a factorisation's chain, beside an update on
-// another stream.
+// C = alpha A B + beta C inside a factorisation, beside another stream's
+// kernels.
 template <class T>
 void gemm_chain(hipStream_t s, int64_t m, int64_t n, int64_t k, T alpha, const T *A, int64_t lda, const T *B,
                 int64_t ldb, T beta, T *C, int64_t ldc);
@@ -149,13 +149,14 @@ int tri_block(int64_t n);
 int64_t tri_inverse_elems(int64_t n);
 template <class T>
 void tri_inverse_build(hipStream_t s, bool lower, bool trans, bool unit, int64_t n, const T *A, int64_t lda, T *W);
-// tri_inverse_solve_to leaves the solution in X (not B) and B updated.
+// tri_inverse_solve_to leaves the solution in X (not B) and B updated.  `chain`:
+// inside a factorisation, beside another stream's kernels (gemm_chain).
 template <class T>
 void tri_inverse_solve_to(hipStream_t s, bool lower, bool trans, int64_t n, int64_t nrhs, const T *A, int64_t lda,
-                          const T *W, T *B, int64_t ldb, T *X, int64_t ldx);
+                          const T *W, T *B, int64_t ldb, T *X, int64_t ldx, bool chain = false);
 template <class T>
 void tri_inverse_solve(hipStream_t s, bool lower, bool trans, int64_t n, int64_t nrhs, const T *A, int64_t lda,
-                       const T *W, T *B, int64_t ldb);
+                       const T *W, T *B, int64_t ldb, bool chain = false);
 
 // LU with partial pivoting, in place; writes d_ipiv[0..n) and *d_info.
 template <class T>

@@ -1533,7 +1533,7 @@ void trailing_update(hipStream_t s, bool bf16, int64_t m, int64_t n, int64_t k, 
     if (sharing)
         gemm_sharing<T>(s, m, n, k, T(-1), L21, lda, U12, lda, T(1), A22, lda, aux_gemm_lds_footprint<T>());
     else
-        gemm(s, false, false, m, n, k, T(-1), L21, lda, U12, lda, T(1), A22, lda);
+        gemm_chain<T>(s, m, n, k, T(-1), L21, lda, U12, lda, T(1), A22, lda);
 }
 
 template <class T>
@@ -1661,14 +1661,14 @@ void getrf_impl(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_ipiv, in
             LMX_HIP(hipStreamWaitEvent(aux, evE, 0));
         }
         if (trail > 0) {
-            tri_inverse_solve<T>(s, true, false, nbw, narrow, A11, lda, W, A12, lda);
+            tri_inverse_solve<T>(s, true, false, nbw, narrow, A11, lda, W, A12, lda, true);
             trailing_update<T>(s, bf16, trail, narrow, nbw, A11 + (int64_t)nbw * lda, lda, A12,
                                A12 + (int64_t)nbw * lda, false);
         }
         // beside panels the kernel with the small LDS footprint
         gather_rows_deferred<T>(aux, A, lda, 0, k0, k0, N, pairs, np, !ahead);
         if (trail > narrow) {
-            tri_inverse_solve<T>(aux, true, false, nbw, trail - narrow, A11, lda, W, A12 + narrow, lda);
+            tri_inverse_solve<T>(aux, true, false, nbw, trail - narrow, A11, lda, W, A12 + narrow, lda, true);
             // at most two GEMM workgroups per CU, so every CU keeps room for
             // a panel workgroup of the caller's stream
             trailing_update<T>(aux, bf16, trail, trail - narrow, nbw, A11 + (int64_t)nbw * lda, lda, A12 + narrow,

@@ -575,8 +575,12 @@ void diag_copy(hipStream_t s, bool mt, bool mlower, int n, int bw, int nbw, cons
 // GEMM otherwise.
 template <class T>
 void apply_block(hipStream_t s, int64_t rows, int64_t k, int64_t nrhs, T alpha, const T *M, int64_t ldm, bool mtrans,
-                 const T *x, int64_t ldx, bool accumulate, T *out, int64_t ldo) {
+                 const T *x, int64_t ldx, bool accumulate, T *out, int64_t ldo, bool chain) {
     if (rows <= 0) return;
+    if (chain && !mtrans && nrhs > 8) {
+        gemm_chain<T>(s, rows, nrhs, k, alpha, M, ldm, x, ldx, accumulate ? T(1) : T(0), out, ldo);
+        return;
+    }
     if (mtrans || nrhs > 8) {
         gemm(s, mtrans, false, rows, nrhs, k, alpha, M, ldm, x, ldx, accumulate ? T(1) : T(0), out, ldo);
         return;
@@ -693,7 +697,7 @@ void tri_inverse_build(hipStream_t s, bool lower, bool trans, bool unit, int64_t
 // the first one's X to the second and needs no copies between.
 template <class T>
 void tri_inverse_solve_to(hipStream_t s, bool lower, bool trans, int64_t n, int64_t nrhs, const T *A, int64_t lda,
-                          const T *W, T *B, int64_t ldb, T *X, int64_t ldx) {
+                          const T *W, T *B, int64_t ldb, T *X, int64_t ldx, bool chain) {
     if (n <= 0 || nrhs <= 0) return;
     if (n > INT32_MAX / 2 || nrhs > INT32_MAX / 2) fail_arg("trsm: dimension too large");
     TimedRegion tr("trsm", s, (double)n * (double)n * (double)nrhs);
@@ -703,11 +707,12 @@ void tri_inverse_solve_to(hipStream_t s, bool lower, bool trans, int64_t n, int6
         const int b = mlower ? bi : nbw - 1 - bi;
         const int64_t j0 = (int64_t)b * bw, nj = std::min<int64_t>(bw, n - j0);
         apply_block<T>(s, nj, nj, nrhs, T(1), W + (int64_t)b * bw * bw, bw, false, B + j0 * ldb, ldb, false,
-                       X + j0 * ldx, ldx);
+                       X + j0 * ldx, ldx, chain);
         const int64_t i0 = mlower ? j0 + nj : 0, ni = mlower ? n - (j0 + nj) : j0;
         if (ni > 0) {
             const T *Mb = mt ? A + j0 * lda + i0 : A + i0 * lda + j0;
-            apply_block<T>(s, ni, nj, nrhs, T(-1), Mb, lda, mt, X + j0 * ldx, ldx, true, B + i0 * ldb, ldb);
+            apply_block<T>(s, ni, nj, nrhs, T(-1), Mb, lda, mt, X + j0 * ldx, ldx, true, B + i0 * ldb, ldb,
+                           chain);
         }
     }
 }
@@ -715,11 +720,11 @@ void tri_inverse_solve_to(hipStream_t s, bool lower, bool trans, int64_t n, int6
 // The same in place on B.
 template <class T>
 void tri_inverse_solve(hipStream_t s, bool lower, bool trans, int64_t n, int64_t nrhs, const T *A, int64_t lda,
-                       const T *W, T *B, int64_t ldb) {
+                       const T *W, T *B, int64_t ldb, bool chain) {
     if (n <= 0 || nrhs <= 0) return;
     Scratch sX((size_t)n * nrhs * sizeof(T), s);
     T *X = sX.as<T>();
-    tri_inverse_solve_to<T>(s, lower, trans, n, nrhs, A, lda, W, B, ldb, X, nrhs);
+    tri_inverse_solve_to<T>(s, lower, trans, n, nrhs, A, lda, W, B, ldb, X, nrhs, chain);
     hipLaunchKernelGGL(copy_rows_kernel<T>, dim3((unsigned)cdiv(n * nrhs, 256)), dim3(256), 0, s, X, nrhs, B, ldb, n,
                        (int)nrhs);
     LMX_LAUNCH_CHECK();
@@ -790,13 +795,13 @@ template void trsm_left<float>(hipStream_t, bool, bool, bool, int64_t, int64_t, 
 template void tri_inverse_build<double>(hipStream_t, bool, bool, bool, int64_t, const double *, int64_t, double *);
 template void tri_inverse_build<float>(hipStream_t, bool, bool, bool, int64_t, const float *, int64_t, float *);
 template void tri_inverse_solve_to<double>(hipStream_t, bool, bool, int64_t, int64_t, const double *, int64_t,
-                                       const double *, double *, int64_t, double *, int64_t);
+                                       const double *, double *, int64_t, double *, int64_t, bool);
 template void tri_inverse_solve<double>(hipStream_t, bool, bool, int64_t, int64_t, const double *, int64_t,
-                                        const double *, double *, int64_t);
+                                        const double *, double *, int64_t, bool);
 template void tri_inverse_solve_to<float>(hipStream_t, bool, bool, int64_t, int64_t, const float *, int64_t,
-                                       const float *, float *, int64_t, float *, int64_t);
+                                       const float *, float *, int64_t, float *, int64_t, bool);
 template void tri_inverse_solve<float>(hipStream_t, bool, bool, int64_t, int64_t, const float *, int64_t,
-                                       const float *, float *, int64_t);
+                                       const float *, float *, int64_t, bool);
 template void trsm_right<double>(hipStream_t, bool, bool, bool, int64_t, int64_t, const double *, int64_t, double *,
                                  int64_t);
 template void trsm_right<float>(hipStream_t, bool, bool, bool, int64_t, int64_t, const float *, int64_t, float *,
