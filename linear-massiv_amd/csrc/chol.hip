@@ -443,13 +443,13 @@ void diag_block(hipStream_t s, bool bf16, int64_t kb, T *A11, int64_t lda, int64
 // those beyond it and block column b's panel, which the caller's stream has
 // no more use for).
 // The panel below a diagonal block is L21 = A21 L11^{-T}: one GEMM into
-// scratch. Both updates read it there, and the auxiliary stream copies it
-// to its place in A, which nothing else reads or writes until the end: with
-// the copy on the caller's stream (6 us and a launch gap a block, 31 blocks
-// at n = 8192) FP64 n = 8192 took 9.40
-// against 9.33 ms, the mixed solve at n = 4096 3.54 against 3.50 ms. Two
-// such blocks, used in turn: when block b + 1's panel is formed, block b's is still being read,
-// block b - 1's no longer (done(b - 1) has been waited for).
+// scratch.  Both updates read it there, and the auxiliary stream copies it to
+// its place in A, which nothing else reads or writes until the end: with the
+// copy on the caller's stream (6 us and a launch gap a block, 31 blocks at
+// n = 8192) FP64 n = 8192 took 9.40 against 9.33 ms, the mixed solve at
+// n = 4096 3.54 against 3.50 ms.  Two such blocks, used in turn: when block
+// b + 1's panel is formed, block b's is still being read, block b - 1's no
+// longer (done(b - 1) has been waited for).
 template <class T>
 void potrf_lookahead(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_info, bool bf16) {
     constexpr int64_t nb = BLK;
@@ -484,7 +484,7 @@ void potrf_lookahead(hipStream_t s, int64_t n, T *A, int64_t lda, int32_t *d_inf
         T *X = (k0 / nb) % 2 ? sy.as<T>() : sx.as<T>();
         diag_block<T>(s, bf16, kb, A11, lda, k0, d_info, WT, tmp);
         if (rest > 0) gemm_chain<T>(s, rest, kb, kb, T(1), A21, lda, WT, BLK, T(0), X, kb);
-        // The trailing SYRK may start once the panel is in place: it and
+        // The trailing SYRK may start once the panel is formed in X: it and
         // the next block column's update below touch different elements.
         // Recording `ready` here keeps the event markers out of the gap
         // between that update and the next diagonal kernel.

@@ -664,8 +664,8 @@ __global__ __launch_bounds__(64 * KS_WAVES) void gemm_ksplit_kernel(int m, int n
 // Operands as stored, a k-contiguous A costs 16 lines a load and B two, so the
 // tile is wide (64 x 128: 67 TF at 8192^3, 128 x 64: 60 TF).  No operand needs
 // to be aligned.  FP64 8192^3 20.8 -> 16.4 ms (52.9 -> 67.0 TF), A transposed
-// 24.7 -> 15.7 ms, 1999 x 1001 x 777 with A transposed 90 -> 62 us, 3001 x 2999
-// x 1003 588 -> 351 us.
+// 24.6 -> 16.3 ms, 1999 x 1001 x 777 with A transposed 82 -> 55 us, 3001 x 2999
+// x 1003 586 -> 332 us.
 template <class T, int MT, int NT, bool TA, bool TB, bool VEC>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_direct_kernel(
     int m, int n, int k, T alpha, const T *__restrict__ A, int64_t lda, const T *__restrict__ B, int64_t ldb, T beta,
@@ -1029,11 +1029,12 @@ bool bf16_vec_ok(bool ta, bool tb, int64_t m, int64_t n, int64_t k, const S *A, 
 // transposed in registers (v_perm on pairs) and written as 8-byte runs of k,
 // the lanes of a wave on consecutive k.
 //   For rows aligned to 16 bytes and dimensions along memory that are
-// multiples of 8.  Bound by the matrix cores and LDS: 8192^3 2.43 -> 1.21 ms
-// (453 -> 908 TF) as stored, 1.53 -> 1.05 ms with B transposed, against the
-// 128 x 128 x 32 tiles with 8-byte loads; 4096^3 370 -> 136 - 166 us.  The same
+// multiples of 8.  Bound by the matrix cores and LDS: 8192^3 2.39 -> 1.10 - 1.15
+// ms (460 -> 960 - 1000 TF) as stored, 1.55 -> 1.04 ms with B transposed, against
+// the 128 x 128 x 32 tiles with 8-byte loads; 4096^3 348 -> 136 us.  The same
 // with 128 x 128 tiles, 4 waves of 64 x 64, two workgroups a CU, for outputs
-// that leave CUs without a tile: 2048 x 2048 x 4096 145 -> 82 us.
+// that leave CUs without a tile: 2048 x 2048 x 4096 143 -> 78 us.  Which products
+// take them: bf16_large_tile.
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
 constexpr int BX_K = 64, BX_SK = 72;
